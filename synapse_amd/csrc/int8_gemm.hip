@@ -7,7 +7,10 @@
 // 4 steps (one KC chunk) the i32 accumulators are folded into an f32 tile in
 // that order, so the result is bit-identical to the reference.  Two forms:
 // k_gemm_w8a8_dl (direct global->LDS loads; K a multiple of 128) and
-// k_gemm_w8a8_ws (producer waves staging through registers; any K).
+// k_gemm_w8a8_ws (producer waves staging through registers; any K).  With
+// WHOLE both keep one exact i32 sum over all of K and apply the epilogue
+// once, as the M <= 16 rows do: the rows of a prompt then equal those of the
+// decode step bit for bit.
 //
 // Operands: activations int8 [M, ldx] row-major; weights in the 64-row panel
 // layout (linear.hpp), so a 128-byte K step of a panel is 8 contiguous 1 KiB
@@ -44,7 +47,7 @@ template <int TM> constexpr int w_stage() { return (TM + WBN) * WLD; }  // bytes
 
 typedef int i32x16 __attribute__((ext_vector_type(16)));
 
-template <int TM>
+template <int TM, bool WHOLE>
 __global__ void __launch_bounds__(TM * 2 + 256)
     k_gemm_w8a8_ws(const int8_t *__restrict__ xq, int ldx, const float *__restrict__ sx, int M,
                    const i32x4 *__restrict__ W, const float *__restrict__ ws, int N, int C,
@@ -186,7 +189,7 @@ __global__ void __launch_bounds__(TM * 2 + 256)
       if (kk + 1 < WCH / 2) read(t, kk + 1, (kk + 1) & 1);
       mma(kk & 1);
     }
-    if (((t + 1) & 3) == 0 || t + 1 == nsteps) fold();
+    if ((!WHOLE && ((t + 1) & 3) == 0) || t + 1 == nsteps) fold();
     __syncthreads();
   }
 #pragma unroll
@@ -230,7 +233,7 @@ template <int TM, int TN, int NS> constexpr size_t dl_lds_bytes() {
   return (size_t)NS * dl_stage<TM, TN>() + TM * sizeof(float);
 }
 
-template <int TM, int TN, int NS, int WR, bool DF>
+template <int TM, int TN, int NS, int WR, bool DF, bool WHOLE = false>
 __global__ void __launch_bounds__(128 * WR)
     k_gemm_w8a8_dl(const int8_t *__restrict__ xq, int ldx, const float *__restrict__ sx, int M,
                    const i32x4 *__restrict__ W, const float *__restrict__ ws, int N, int C,
@@ -238,6 +241,7 @@ __global__ void __launch_bounds__(128 * WR)
   constexpr int NWAVE = 2 * WR, WM = TM / WR, WN = TN / 2, MT = WM / 32, NT = WN / 32;
   constexpr int LA = TM / 8 / NWAVE, LB = TN / 8 / NWAVE;  // direct loads per wave and step
   static_assert(LA * NWAVE * 8 == TM && LB * NWAVE * 8 == TN, "whole loads per wave");
+  static_assert(!(DF && WHOLE), "one accumulator set without the chunk folds");
   constexpr int A_BYTES = TM * 128, STAGE = dl_stage<TM, TN>(), AFTER = LA + LB;
   extern __shared__ __attribute__((aligned(16))) int8_t dlds[];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -431,7 +435,7 @@ __global__ void __launch_bounds__(128 * WR)
     };
     for (int t = 0; t < nsteps; t++) {
       step(t, 0, P0{}, NoFold{});
-      if (((t + 1) & 3) == 0 || t + 1 == nsteps) fold1();
+      if ((!WHOLE && ((t + 1) & 3) == 0) || t + 1 == nsteps) fold1();
     }
   } else {
     const int nfull = nsteps >> 2;
@@ -475,20 +479,39 @@ __global__ void __launch_bounds__(128 * WR)
     }
 }
 
-template <int TM, int TN, int NS, int WR, bool DF>
+template <int TM, int TN, int NS, int WR, bool DF, bool WHOLE = false>
 static syn_status_t launch_w8a8_dl(const int8_t *xq, size_t ldx, const float *sx, size_t M,
                                    const void *W, const float *ws, size_t N, int C, float *y,
                                    size_t ldy, hipStream_t s) {
   static bool attr_set = false;  // more than the default 64 KiB of dynamic LDS
   constexpr size_t shm = dl_lds_bytes<TM, TN, NS>();
   if (!attr_set) {
-    SYN_HIP(hipFuncSetAttribute((const void *)k_gemm_w8a8_dl<TM, TN, NS, WR, DF>,
+    SYN_HIP(hipFuncSetAttribute((const void *)k_gemm_w8a8_dl<TM, TN, NS, WR, DF, WHOLE>,
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm));
     attr_set = true;
   }
   const dim3 grid((unsigned)cdiv(N, TN), (unsigned)cdiv(M, TM));
-  SYN_LAUNCH((k_gemm_w8a8_dl<TM, TN, NS, WR, DF>), grid, dim3(128 * WR), shm, s, xq, (int)ldx, sx, (int)M,
+  SYN_LAUNCH((k_gemm_w8a8_dl<TM, TN, NS, WR, DF, WHOLE>), grid, dim3(128 * WR), shm, s, xq, (int)ldx, sx, (int)M,
              (const i32x4 *)W, ws, (int)N, C, y, (int)ldy);
+  SYN_LAUNCH_CHECK();
+  return SYN_OK;
+}
+
+// two LDS stages of 128-byte K steps exceed the default 64 KiB
+template <int TM, bool WHOLE>
+static syn_status_t launch_w8a8_ws(const int8_t *xq, size_t ldx, const float *sx, size_t M,
+                                   const void *W, const float *ws, size_t N, int C, float *y,
+                                   size_t ldy, hipStream_t s) {
+  static bool attr_set = false;
+  const dim3 grid((unsigned)cdiv(N, WBN), (unsigned)cdiv(M, TM));
+  const size_t shm = 2 * (size_t)w_stage<TM>() + TM * sizeof(float);
+  if (!attr_set) {
+    SYN_HIP(hipFuncSetAttribute((const void *)k_gemm_w8a8_ws<TM, WHOLE>,
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm));
+    attr_set = true;
+  }
+  hipLaunchKernelGGL((k_gemm_w8a8_ws<TM, WHOLE>), grid, dim3(TM * 2 + 256), shm, s, xq, (int)ldx,
+                     sx, (int)M, (const i32x4 *)W, ws, (int)N, C, y, (int)ldy);
   SYN_LAUNCH_CHECK();
   return SYN_OK;
 }
@@ -537,31 +560,28 @@ syn_status_t launch_gemm_w8a8(const int8_t *xq, size_t ldx, const float *sx, siz
   }
   // otherwise 256-row tiles, or 128-row tiles when the larger ones cannot
   // fill the GPU
-  // two LDS stages of 128-byte K steps exceed the default 64 KiB
-  static bool attr_set[2] = {false, false};
-  if (cdiv(M, 256) * cdiv(N, WBN) >= 256) {
-    dim3 grid((unsigned)cdiv(N, WBN), (unsigned)cdiv(M, 256));
-    const size_t shm = 2 * (size_t)w_stage<256>() + 256 * sizeof(float);
-    if (!attr_set[0]) {
-      SYN_HIP(hipFuncSetAttribute((const void *)k_gemm_w8a8_ws<256>,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm));
-      attr_set[0] = true;
-    }
-    hipLaunchKernelGGL(k_gemm_w8a8_ws<256>, grid, dim3(768), shm, s, xq, (int)ldx, sx, (int)M,
-                       (const i32x4 *)W, ws, (int)N, C, y, (int)ldy);
-  } else {
-    dim3 grid((unsigned)cdiv(N, WBN), (unsigned)cdiv(M, 128));
-    const size_t shm = 2 * (size_t)w_stage<128>() + 128 * sizeof(float);
-    if (!attr_set[1]) {
-      SYN_HIP(hipFuncSetAttribute((const void *)k_gemm_w8a8_ws<128>,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm));
-      attr_set[1] = true;
-    }
-    hipLaunchKernelGGL(k_gemm_w8a8_ws<128>, grid, dim3(512), shm, s, xq, (int)ldx, sx, (int)M,
-                       (const i32x4 *)W, ws, (int)N, C, y, (int)ldy);
+  if (cdiv(M, 256) * cdiv(N, WBN) >= 256)
+    return launch_w8a8_ws<256, false>(xq, ldx, sx, M, W, ws, N, C, y, ldy, s);
+  return launch_w8a8_ws<128, false>(xq, ldx, sx, M, W, ws, N, C, y, ldy, s);
+}
+
+syn_status_t launch_gemm_w8a8_whole(const int8_t *xq, size_t ldx, const float *sx, size_t M,
+                                    const void *W, const float *ws, size_t N, int C, float *y,
+                                    size_t ldy, hipStream_t s) {
+  if (ldx % 16) {
+    set_error("activation row stride must be a multiple of 16 bytes");
+    return SYN_ERR_SHAPE_MISMATCH;
   }
-  SYN_LAUNCH_CHECK();
-  return SYN_OK;
+  if (C > kWholeMaxChunks) {  // |sum| <= 128 * 128 * 16 C stays below 2^31
+    set_error("INT8 GEMM: K too long for one 32-bit sum");
+    return SYN_ERR_INVALID_ARG;
+  }
+  if (C % 8 == 0 && (uintptr_t)xq % 16 == 0 && M * ldx < ((size_t)1 << 31)) {
+    if (cdiv(M, 128) * cdiv(N, 128) >= 256)
+      return launch_w8a8_dl<128, 128, 2, 4, false, true>(xq, ldx, sx, M, W, ws, N, C, y, ldy, s);
+    return launch_w8a8_dl<64, 64, 4, 2, false, true>(xq, ldx, sx, M, W, ws, N, C, y, ldy, s);
+  }
+  return launch_w8a8_ws<128, true>(xq, ldx, sx, M, W, ws, N, C, y, ldy, s);
 }
 
 }  // namespace syn

@@ -76,6 +76,13 @@ syn_status_t launch_gemm_w8a8(const int8_t *xq, size_t ldx, const float *sx, siz
                               const void *W, const float *ws, size_t N, int C, float *y,
                               size_t ldy, hipStream_t s);
 
+// the same product with one i32 sum over the whole K and a single epilogue
+// (f32(acc) * sx) * ws, the M <= 16 form at any M
+constexpr int kWholeMaxChunks = 8191;  // 16-byte K chunks of an exact 32-bit sum
+syn_status_t launch_gemm_w8a8_whole(const int8_t *xq, size_t ldx, const float *sx, size_t M,
+                                    const void *W, const float *ws, size_t N, int C, float *y,
+                                    size_t ldy, hipStream_t s);
+
 // host-side reference quantizers (used at load time)
 void host_minmax_scales(const float *w, size_t ch, size_t chsz, float *scales);
 void host_quantize_weights_nk(const float *w, const float *scales, size_t n, size_t k,
