@@ -20,6 +20,7 @@
 #include "decode_fused.hpp"
 #include "kquant.hpp"
 #include "lds_dma.hpp"
+#include "rows_gemm.hpp"
 
 namespace syn {
 
@@ -880,7 +881,15 @@ __global__ void __launch_bounds__(256)
 // power of two whose inverse lands in *rowmul (m floats after the rows), in
 // the k_gemm_kqr Q4_0 chunk order if perm8
 size_t f16_rows_bytes(size_t m, size_t k) {
-  return round_up(m * round_up(k, PGK) * 2, 256) + m * sizeof(float);
+  // also rows_frag_bytes(m, k, false), whose rows are whole 32-row tiles
+  return round_up(round_up(m, 32) * round_up(k, PGK) * 2, 256) + round_up(m, 32) * sizeof(float);
+}
+static syn_status_t ensure_rows(size_t need, DevBuf &xh, size_t &xh_bytes) {
+  if (xh_bytes >= need) return SYN_OK;
+  SYN_HIP(hipDeviceSynchronize());
+  SYN_TRY(xh.alloc(need));
+  xh_bytes = need;
+  return SYN_OK;
 }
 static syn_status_t to_f16_rows(size_t m, size_t k, const float *d_x, size_t ldx, DevBuf &xh,
                                 size_t &xh_bytes, bool perm8, float **rowmul, hipStream_t s,
@@ -891,12 +900,7 @@ static syn_status_t to_f16_rows(size_t m, size_t k, const float *d_x, size_t ldx
   }
   if (m > 0x7fffffffu) return SYN_ERR_INVALID_ARG;
   const size_t ldh = round_up(k, PGK);  // zero-padded to whole K steps
-  const size_t need = f16_rows_bytes(m, k);
-  if (xh_bytes < need) {
-    SYN_HIP(hipDeviceSynchronize());
-    SYN_TRY(xh.alloc(need));
-    xh_bytes = need;
-  }
+  SYN_TRY(ensure_rows(f16_rows_bytes(m, k), xh, xh_bytes));
   *rowmul = reinterpret_cast<float *>(xh.as<unsigned char>() + round_up(m * ldh * 2, 256));
   hipLaunchKernelGGL(k_f32_to_f16, dim3((unsigned)m), dim3(256), 0, s, d_x, (int)ldx,
                      xh.as<_Float16>(), (int)ldh, *rowmul, (int)k, perm8 ? 1 : 0, zero_y0,
@@ -942,6 +946,21 @@ static syn_status_t kq_gemm_f16(int fmt, bool exact, const u32x4 *W, const uint1
                                 hipStream_t s) {
   const size_t ldh = round_up(k, PGK);
   const int steps = (int)cdiv(k, PGK);
+  if (rows_gemm_fits(fmt, exact, m, n, k)) {
+    RowsGemm g;
+    g.fmt = fmt;
+    g.W = W;
+    g.Wd = Wd;
+    g.blocks = blocks;
+    g.n = n;
+    g.k = k;
+    // K splits add into rows that the conversion clears 16 bytes at a time
+    const bool can_split = ldy % 4 == 0 && reinterpret_cast<uintptr_t>(d_y) % 16 == 0;
+    const int kz = can_split ? rows_gemm_splits(g, m) : 1;
+    SYN_TRY(ensure_rows(f16_rows_bytes(m, k), xh, xh_bytes));
+    SYN_TRY(launch_rows_frag(fmt, d_x, ldx, m, k, false, xh.p, kz > 1 ? d_y : nullptr, ldy, n, s));
+    return launch_rows_gemm(g, xh.p, m, kz, d_y, ldy, s);
+  }
   // dynamic-LDS attribute set per kernel: k_gemm_kq5 0-3 and 8, k_gemm_kqr
   // 10, k_gemm_kq2 11-15 (256-row tiles) and 16-20 (128-row tiles)
   static bool attr[21] = {};

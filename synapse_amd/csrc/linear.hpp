@@ -132,6 +132,10 @@ struct QLinearQ4_0 {
   // activations rounded once to f16, f32 accumulation
   syn_status_t gemm(size_t m, const float *d_x, size_t ldx, float *d_y, size_t ldy,
                     hipStream_t s);
+  // 7 to 16 rows on the matrix cores with f32 accuracy (rows_gemm.hip)
+  syn_status_t gemm_split(size_t m, const float *d_x, size_t ldx, float *d_y, size_t ldy,
+                          hipStream_t s);
+  syn_status_t ensure_split(size_t m);
   // the GEMM decodes the scales as IEEE f16 values: not for halved subnormals
   bool gemm_ok() const { return !(rs_f16_scales && has_subnormal_scale); }
 };

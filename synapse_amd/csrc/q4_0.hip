@@ -14,6 +14,7 @@
 #include <vector>
 
 #include "linear.hpp"
+#include "rows_gemm.hpp"
 #include "split_k.hpp"
 
 namespace syn {
@@ -337,6 +338,13 @@ syn_status_t QLinearQ4_0::gemv(size_t m, const float *d_x, size_t ldx, float *d_
                                hipStream_t s) {
   if (m == 0 || n == 0 || k == 0) return SYN_OK;
   if (m > 16 && gemm_ok() && ldx % 4 == 0) return gemm(m, d_x, ldx, d_y, ldy, s);
+  // 9 to 16 rows: two GEMV launches read the weights twice (3072 -> 8192: 25-37
+  // us against 12 on the matrix cores, 4096 -> 1024 16-18 against 12.5, 2048
+  // -> 2048 13-15 against 9).  7 and 8 rows only on large matrices (8 rows,
+  // 3072 -> 8192 18.6 against 12, 14336 -> 4096 38 against 30; 4096 -> 1024
+  // 9.0 against 12.5)
+  if (gemm_ok() && ldx % 4 == 0 && m <= 16 && (m >= 9 || (m >= 7 && n * k >= 24000000)))
+    return gemm_split(m, d_x, ldx, d_y, ldy, s);
   const float sub = rs_f16_scales ? 0.5f : 1.0f;
   // "chunks" here are 32-element blocks; a K slice holds whole blocks.  One
   // launch per block of up to 8 rows: a K split finishes in place (split_k.hpp)
@@ -357,6 +365,29 @@ syn_status_t QLinearQ4_0::gemv(size_t m, const float *d_x, size_t ldx, float *d_
     }
     SYN_LAUNCH_CHECK();
   }
+  return SYN_OK;
+}
+
+syn_status_t QLinearQ4_0::gemm_split(size_t m, const float *d_x, size_t ldx, float *d_y,
+                                     size_t ldy, hipStream_t s) {
+  RowsGemm g;
+  g.fmt = SYN_HIP_FMT_Q4_0;
+  g.W = nib.p;
+  g.Wd = sc.as<uint16_t>();
+  g.blocks = blocks;
+  g.n = n;
+  g.k = k;
+  SYN_TRY(ensure_split(m));
+  SYN_TRY(launch_rows_frag(g.fmt, d_x, ldx, m, k, true, xh.p, nullptr, 0, 0, s));
+  return launch_rows_gemm_split(g, xh.p, m, 1, d_y, ldy, 0, s);
+}
+
+syn_status_t QLinearQ4_0::ensure_split(size_t m) {
+  const size_t need = rows_frag_bytes(m, k, true);
+  if (xh_bytes >= need) return SYN_OK;
+  SYN_HIP(hipDeviceSynchronize());  // the old buffer may still be read by queued work
+  SYN_TRY(xh.alloc(need));
+  xh_bytes = need;
   return SYN_OK;
 }
 
@@ -384,6 +415,7 @@ syn_status_t QLinearQ4_0::gemv_parts(const float *d_x, float *d_y, PartRows *out
 syn_status_t QLinearQ4_0::prepare(size_t max_m) {
   const GemvPlan p = make_gemv_plan(n, (size_t)blocks, false);
   if (p.ksplit > 1) SYN_TRY(sk.ensure(p.panels, 8, p.ksplit));
+  if (max_m >= 7) SYN_TRY(ensure_split(std::min<size_t>(16, max_m)));
   const size_t need = (size_t)p.ksplit * std::min<size_t>(8, max_m) * (size_t)p.panels * 64;
   if (p.ksplit > 1 && part_elems < need) {
     part_elems = need;

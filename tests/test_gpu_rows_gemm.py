@@ -1,0 +1,112 @@
+"""The few-row quantized GEMM against float64 products of the dequantized
+weights, at the edges of its tiles and of its dispatch rule.
+
+Bounds, per element and relative to sum |x w|: one f16 rounding (2^-11) of
+each activation and each weight, plus f32 sums, stay below 2^-10 (1 + 2^-4).
+Split Q4_0 (7 to 16 rows): the weights are exact, an activation's two halves
+leave at most 2^-22 of it, the product of the remainders that is not formed
+2^-22, and the f32 sums of at most K / 16 + 16 partial sums 2^-24 each."""
+import numpy as np
+import pytest
+
+from synapse_amd import hip
+
+pytestmark = pytest.mark.gpu
+
+EL = {hip.FMT_Q4_0: 32, hip.FMT_Q8_0: 32, hip.FMT_Q4_K: 256, hip.FMT_Q6_K: 256}
+NAME = {hip.FMT_Q4_0: "q4_0", hip.FMT_Q8_0: "q8_0", hip.FMT_Q4_K: "q4_k", hip.FMT_Q6_K: "q6_k"}
+
+
+@pytest.fixture(scope="module", autouse=True)
+def gpu():
+    hip.init(0)
+
+
+def _linear(fmt, n, k, seed):
+    """a handle and its float64 weights"""
+    rng = np.random.default_rng(seed)
+    w = rng.standard_normal((n, k)).astype(np.float32) * 0.05
+    if fmt == hip.FMT_Q4_0:
+        raw = rng.integers(0, 256, (n * k // 32, 18), dtype=np.uint8)
+        d = (rng.random(n * k // 32) * 0.01 + 1e-3).astype(np.float16)
+        raw[:, :2] = d.view(np.uint8).reshape(-1, 2)
+        q = np.empty((n * k // 32, 32))
+        q[:, 0::2], q[:, 1::2] = raw[:, 2:] & 15, raw[:, 2:] >> 4
+        return (hip.QLinear.q4_0(raw.reshape(-1), n, k),
+                ((q - 8) * d.astype(np.float64)[:, None]).reshape(n, k))
+    blocks = hip.kquant_encode(fmt, w)
+    return (hip.QLinear.gguf(fmt, blocks, n, k),
+            hip.kquant_decode(fmt, blocks).astype(np.float64).reshape(n, k))
+
+
+def _check(lin, w, x, split):
+    m, k = x.shape
+    got = lin.forward(x).astype(np.float64)
+    want = x.astype(np.float64) @ w.T
+    size = np.abs(x).astype(np.float64) @ np.abs(w).T
+    bound = 2.0**-21 + (k / 16 + 16) * 2.0**-24 if split else 2.0**-10 * (1 + 2.0**-4)
+    worst = float((np.abs(got - want) / size).max())
+    print(NAME[lin.fmt], "m", m, "n", w.shape[0], "k", k, "worst", worst, "bound", bound, flush=True)
+    assert worst <= bound, (m, worst, bound)
+    return worst
+
+
+# rows: one and two tiles of 32, one and two passes of 64, the rule's lines
+# at 128 / 129 and 256 / 257; K: one step, an odd number of half steps, fewer
+# and more steps than waves, a K split; N: a part of a panel, several panels
+@pytest.mark.parametrize("fmt", sorted(EL), ids=lambda f: NAME[f])
+@pytest.mark.parametrize("n,k", [(36, 256), (100, 512), (64, 2304), (320, 4096)])
+def test_rows_gemm_edges(fmt, n, k):
+    lin, w = _linear(fmt, n, k, n + k)
+    rng = np.random.default_rng(k)
+    x = rng.standard_normal((260, k)).astype(np.float32)
+    x[:, rng.integers(0, k, 3)] *= 50
+    x[3] *= 1e-7
+    x[5] *= 1e6
+    for m in (9, 16, 17, 31, 32, 33, 64, 65, 127, 128, 129, 256, 257):
+        _check(lin, w, x[:m], fmt == hip.FMT_Q4_0 and m <= 16)
+    lin.close()
+
+
+@pytest.mark.parametrize("fmt", [hip.FMT_Q4_0, hip.FMT_Q8_0], ids=lambda f: NAME[f])
+@pytest.mark.parametrize("k", [32, 96, 1056])
+def test_rows_gemm_half_step_tail(fmt, k):
+    lin, w = _linear(fmt, 72, k, k)
+    x = np.random.default_rng(k).standard_normal((40, k)).astype(np.float32)
+    for m in (9, 16, 17, 40):
+        _check(lin, w, x[:m], fmt == hip.FMT_Q4_0 and m <= 16)
+    lin.close()
+
+
+def test_split_rows_seven_and_eight():
+    # 7 and 8 rows take the split form from 24e6 weights on; both sides of the line
+    for n, k in ((8192, 3072), (1024, 2048)):
+        lin, w = _linear(hip.FMT_Q4_0, n, k, 3)
+        x = np.random.default_rng(5).standard_normal((8, k)).astype(np.float32)
+        for m in (6, 7, 8):
+            _check(lin, w, x[:m], True)
+        lin.close()
+
+
+def test_split_rows_extremes():
+    # a row of subnormals, a zero row, rows at the ends of the f32 range; a
+    # NaN or an infinity stays in its own row
+    k, n = 256, 64
+    lin, w = _linear(hip.FMT_Q4_0, n, k, 8)
+    x = np.random.default_rng(9).standard_normal((12, k)).astype(np.float32)
+    x[0] *= np.float32(1e-41)
+    x[1] = 0
+    x[2] *= np.float32(1e-30)
+    x[3] *= np.float32(1e30)
+    x[4, 7] = np.inf
+    x[5, 9] = np.nan
+    got = lin.forward(x)
+    with np.errstate(invalid="ignore"):
+        want = x.astype(np.float64) @ w.T
+    assert not got[1].any()
+    assert np.isnan(got[5]).all() and not np.isfinite(got[4]).any()
+    for r in (0, 2, 3, 6, 7, 8, 9, 10, 11):
+        size = np.abs(x[r]).astype(np.float64) @ np.abs(w).T
+        # subnormal outputs round to 2^-149
+        assert (np.abs(got[r] - want[r]) <= 1e-6 * size + 2.0**-148).all(), r
+    lin.close()
