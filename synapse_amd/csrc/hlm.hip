@@ -34,6 +34,7 @@
 #include "f32_ops.hpp"
 #include "head_f32.hpp"
 #include "klm_fused.hpp"
+#include "hlm_prefill.hpp"
 #include "layer_ops.hpp"
 #include "linear.hpp"
 #include "liv_conv.hpp"
@@ -359,10 +360,15 @@ struct syn_hip_hlm_s {
       d.x = hbuf.as<float>();
       SYN_TRY(kqf_gemv(Ly.down, fp_down, KQF_PRO_NONE, d, r, zero_after, nzero, s));
     }
-    HeadIn hin;  // the tied f32 lm_head of rmsnorm(r)
-    hin.fx = r;
+    return head_fused(s);
+  }
+
+  // the tied f32 lm_head of rmsnorm(r) with its top-2, then the argmax
+  syn_status_t head_fused(hipStream_t s) {
+    HeadIn hin;
+    hin.fx = f_r.as<long long>();
     hin.gain = final_nw.as<float>();
-    hin.eps = eps;
+    hin.eps = c.eps;
     SYN_TRY(launch_head_f32_top2(embed.as<float>(), (int)V, (int)H, hin, logits.as<float>(),
                                  f_pv.as<float>(), f_pi.as<int>(), f_pv2.as<float>(), s));
     return launch_argmax_advance(f_pv.as<float>(), f_pi.as<int>(), f_pv2.as<float>(),
@@ -418,6 +424,118 @@ struct syn_hip_hlm_s {
     SYN_TRY(launch_argmax(logits.as<float>(), (int)V, pv.as<float>(), pi.as<int>(),
                           pv2.as<float>(), st(), history.as<uint32_t>(), mhist.as<float>(), s));
     return launch_step_advance(st(), 1, s);
+  }
+
+  // ---- a prompt's rows (hlm_prefill.hip), from an empty cache; scratch of at
+  // most kRowsMax tokens, kept between prompts
+  static constexpr size_t kRowsMax = 2048;
+  // Below this many tokens the replayed step is the faster form: a layer of
+  // the rows form takes ~65 us at 3-32 tokens, the step ~20 us a token.  LFM2.5
+  // widths, four layers, whole calls: 3 tokens 337 us against 495, 64 tokens
+  // 417 against 9400
+  static constexpr size_t kRowsMin = 3;
+  struct RowsScratch {
+    size_t cap = 0;
+    DevBuf ids, x, part, xf, qrot, attn;
+    size_t part_elems = 0;
+  } rs;
+
+  // the fused step's shapes (Q4_0 with IEEE scales, whole 256s) within the
+  // row kernels' registers and the prompt attention's LDS
+  bool rows_supported() const {
+    return use_fused && fused_ok && H <= (size_t)kHrowsMaxH && I <= (size_t)kHrowsMaxH &&
+           qd <= (size_t)kHrowsMaxH && F <= (size_t)kHrowsMaxF;
+  }
+  static RowsGemm rows_of(const QLinearQ4_0 &q) {
+    RowsGemm g;
+    g.fmt = SYN_HIP_FMT_Q4_0;
+    g.W = q.nib.p;
+    g.Wd = q.sc.as<uint16_t>();
+    g.blocks = q.blocks;
+    g.n = q.n;
+    g.k = q.k;
+    return g;
+  }
+
+  syn_status_t rows_scratch(size_t n) {
+    size_t part = 0, kmax = H;
+    for (auto &Ly : layers)
+      for (QLinearQ4_0 *q : {&Ly.in, &Ly.out, &Ly.qkv, &Ly.o, &Ly.gu, &Ly.down}) {
+        if (!q->n) continue;
+        kmax = std::max(kmax, q->k);
+        part = std::max(part, n * q->n * (size_t)rows_gemm_splits(rows_of(*q), n, true));
+      }
+    if (rs.part_elems < part) {
+      SYN_HIP(hipStreamSynchronize(stream));
+      rs.part_elems = 0;
+      SYN_TRY(rs.part.alloc(part * 4));
+      rs.part_elems = part;
+    }
+    if (rs.cap >= n) return SYN_OK;
+    n = round_up(n, 64);
+    SYN_HIP(hipStreamSynchronize(stream));
+    rs.cap = 0;
+    SYN_TRY(rs.ids.alloc(n * 4));
+    SYN_TRY(rs.x.alloc(n * H * 4));
+    SYN_TRY(rs.xf.alloc(rows_frag_bytes(n, kmax, true)));
+    SYN_TRY(rs.qrot.alloc(n * qd * 4));
+    SYN_TRY(rs.attn.alloc(n * qd * 4));
+    rs.cap = n;
+    return SYN_OK;
+  }
+
+  // rs.part = the fragments in rs.xf times W^T, in at most kz K splits
+  syn_status_t rows_gemm(const QLinearQ4_0 &q, size_t n, int kz, HRows *out) {
+    const RowsGemm g = rows_of(q);
+    kz = std::min(kz, rows_gemm_splits(g, n, true));
+    *out = HRows{rs.part.as<float>(), kz, n * q.n, (int)q.n};
+    return launch_rows_gemm_split(g, rs.xf.p, n, kz, rs.part.as<float>(), q.n, n * q.n, stream);
+  }
+
+  // every layer over ids[0..n) at positions 0.., then the lm_head and argmax
+  // of the last token; the state must be empty.  step: the history slot
+  syn_status_t prefill_rows(const uint32_t *ids, size_t n, int step) {
+    SYN_TRY(rows_scratch(n));
+    SYN_TRY(set_state((int)n - 1, ids[n - 1], step));
+    SYN_HIP(hipMemcpyAsync(rs.ids.p, ids, n * 4, hipMemcpyHostToDevice, stream));
+    const int T = (int)n;
+    float *x = rs.x.as<float>();
+    HRows add;  // the last projection's rows, still to be added to x
+    for (size_t l = 0; l < L; l++) {
+      Layer &Ly = layers[l];
+      SYN_TRY(launch_hrows_norm(x, embed.as<float>(), l == 0 ? rs.ids.as<uint32_t>() : nullptr,
+                                (int)V, add, Ly.attn_nw.as<float>(), c.eps, T, (int)H, rs.xf.p,
+                                stream));
+      HRows p;
+      if (Ly.kind == 0) {
+        SYN_TRY(rows_gemm(Ly.in, n, kRowsMaxSplit, &p));
+        SYN_TRY(launch_hrows_conv(p, Ly.conv_w.as<float>(),
+                                  c.conv_bias ? Ly.conv_b.as<float>() : nullptr, T, (int)I,
+                                  (int)ck, Ly.conv_state.as<float>() + (n & 1) * I * ck, rs.xf.p,
+                                  stream));
+        SYN_TRY(rows_gemm(Ly.out, n, kRowsMaxSplit, &add));
+      } else {
+        SYN_TRY(rows_gemm(Ly.qkv, n, 1, &p));
+        SYN_TRY(launch_qk_norm_rope_kv(p.p, p.ld, T, (int)nh, (int)nkv, (int)hd,
+                                       Ly.q_nw.as<float>(), Ly.k_nw.as<float>(), c.eps,
+                                       rope_cos.as<float>(), rope_sin.as<float>(), nullptr, 0,
+                                       rs.qrot.as<float>(), Ly.kc.as<float>(), Ly.vc.as<float>(),
+                                       (int)S, stream));
+        SYN_TRY(launch_attention_prefill_tol(rs.qrot.as<float>(), Ly.kc.as<float>(),
+                                             Ly.vc.as<float>(), T, (int)nh, (int)nkv, (int)hd,
+                                             (int)S, rs.attn.as<float>(), stream));
+        SYN_TRY(launch_rows_frag(SYN_HIP_FMT_Q4_0, rs.attn.as<float>(), qd, n, qd, true, rs.xf.p,
+                                 nullptr, 0, 0, stream));
+        SYN_TRY(rows_gemm(Ly.o, n, kRowsMaxSplit, &add));
+      }
+      SYN_TRY(launch_hrows_norm(x, nullptr, nullptr, 0, add, Ly.ffn_nw.as<float>(), c.eps, T,
+                                (int)H, rs.xf.p, stream));
+      SYN_TRY(rows_gemm(Ly.gu, n, kRowsMaxSplit, &p));
+      SYN_TRY(launch_hrows_swiglu(p, T, (int)F, rs.xf.p, stream));
+      SYN_TRY(rows_gemm(Ly.down, n, kRowsMaxSplit, &add));
+    }
+    SYN_TRY(launch_hrows_last(x, add, T, (int)H, f_r.as<long long>(), stream));
+    return head_fused(stream);
   }
 
   syn_status_t build_graph() {
@@ -674,7 +792,23 @@ syn_status_t syn_hip_hlm_prefill(syn_hip_hlm_t *m, const uint32_t *ids, size_t n
                                  float *host_logits) {
   SYN_TRY(check_hlm(m));
   if (!ids) return SYN_ERR_NULL_PTR;
-  for (size_t i = 0; i < n; i++)
+  if (n == 0) return SYN_OK;
+  StepState cur;
+  SYN_TRY(m->get_state(&cur));
+  size_t i = 0;
+  // into an empty cache all at once (the rest of a longer prompt, and a
+  // prompt into a filled cache, token by token)
+  if (cur.pos == 0 && n >= m->kRowsMin && n <= m->S && m->rows_supported()) {
+    i = std::min(n, m->kRowsMax);
+    SYN_TRY(m->prefill_rows(ids, i, cur.step + (int)i - 1));
+    if (i == n) {
+      if (host_logits)
+        SYN_HIP(hipMemcpyAsync(host_logits, m->logits.p, m->V * 4, hipMemcpyDeviceToHost,
+                               m->stream));
+      SYN_HIP(hipStreamSynchronize(m->stream));
+    }
+  }
+  for (; i < n; i++)
     SYN_TRY(syn_hip_hlm_decode_one(m, ids[i], i + 1 == n ? host_logits : nullptr));
   return SYN_OK;
 }
@@ -690,10 +824,16 @@ syn_status_t syn_hip_hlm_generate(syn_hip_hlm_t *m, const uint32_t *prompt, size
     set_error("hybrid LM: prompt + generated tokens exceed max_seq");
     return SYN_ERR_INVALID_ARG;
   }
-  for (size_t i = 0; i + 1 < n_prompt; i++) SYN_TRY(syn_hip_hlm_decode_one(m, prompt[i], nullptr));
   // the last prompt token's argmax is the first generated token (step 0)
-  SYN_TRY(m->set_state(cur.pos + (int)n_prompt - 1, prompt[n_prompt - 1], 0));
-  for (size_t i = 0; i < max_new; i++) SYN_TRY(m->run_step());
+  size_t made = 0;
+  if (cur.pos == 0 && n_prompt >= m->kRowsMin && n_prompt <= m->kRowsMax && m->rows_supported()) {
+    SYN_TRY(m->prefill_rows(prompt, n_prompt, 0));
+    made = 1;
+  } else {
+    if (n_prompt > 1) SYN_TRY(syn_hip_hlm_prefill(m, prompt, n_prompt - 1, nullptr));
+    SYN_TRY(m->set_state(cur.pos + (int)n_prompt - 1, prompt[n_prompt - 1], 0));
+  }
+  for (; made < max_new; made++) SYN_TRY(m->run_step());
   SYN_HIP(hipMemcpyAsync(out_tokens, m->history.p, max_new * 4, hipMemcpyDeviceToHost,
                          m->stream));
   if (out_margins)

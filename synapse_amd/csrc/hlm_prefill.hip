@@ -1,0 +1,240 @@
+// The hybrid (LFM2.5) layers over the rows of a prompt.  Token by token a
+// prompt reads every weight and the 268 MB lm_head once per token (~0.15 ms at
+// four layers); here the projections are split-f16 matrix products over all
+// tokens (rows_gemm.hip: as accurate as the step's f32 sums), and the ops
+// between them are one kernel each that sums the product's K splits, computes
+// its rows and writes the next product's activation fragments directly.
+#include "hlm_prefill.hpp"
+#include "rows_frag.hpp"
+
+namespace syn {
+
+namespace {
+
+// columns 8c .. 8c+7 (offset by `off`) of row t
+__device__ __forceinline__ void hrow_get(const HRows &h, int t, int off, int c, float (&v)[8]) {
+  const float *p = h.p + (size_t)t * h.ld + off + 8 * c;
+#pragma unroll
+  for (int i = 0; i < 8; i++) v[i] = 0.0f;
+  for (int z = 0; z < h.kz; z++, p += h.zs) {
+    const float4 a = *reinterpret_cast<const float4 *>(p);
+    const float4 b = *reinterpret_cast<const float4 *>(p + 4);
+    v[0] += a.x; v[1] += a.y; v[2] += a.z; v[3] += a.w;
+    v[4] += b.x; v[5] += b.y; v[6] += b.z; v[7] += b.w;
+  }
+}
+
+template <int NT>
+__device__ __forceinline__ float block_max(float v, float *red) {
+  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < NT / 64; i++) v = fmaxf(v, red[i]);
+  return v;
+}
+
+// scale the thread's chunks tid, tid + NT, .. by the row's power of two and
+// write them (zeros for the padding rows of the last tile)
+template <int NT, int R>
+__device__ __forceinline__ void put_row(float (&v)[R][8], int chunks, float mx, bool real, int m,
+                                        f16x8 *__restrict__ xf, float *__restrict__ rowmul) {
+  float up, down;
+  frag_row_scale(mx, &up, &down);
+  if (threadIdx.x == 0) rowmul[m] = down;
+  const int steps = (8 * chunks + kFragStep - 1) / kFragStep;
+#pragma unroll
+  for (int j = 0; j < R; j++) {
+    const int c = threadIdx.x + NT * j;
+    if (c >= chunks) break;
+#pragma unroll
+    for (int i = 0; i < 8; i++) v[j][i] = real ? v[j][i] * up : 0.0f;
+    frag_put<true, true>(xf, steps, m, c, v[j]);
+  }
+}
+
+constexpr int kNormNT = 256, kNormR = kHrowsMaxH / 8 / kNormNT;
+constexpr int kGluNT = 512, kGluR = kHrowsMaxF / 8 / kGluNT;
+
+// one workgroup per row; row values in registers between the reductions
+__global__ void __launch_bounds__(kNormNT)
+    k_hrows_norm(float *__restrict__ x, const float *__restrict__ embed,
+                 const uint32_t *__restrict__ ids, int vocab, HRows add,
+                 const float *__restrict__ gain, float eps, int T, int H, f16x8 *__restrict__ xf,
+                 float *__restrict__ rowmul) {
+  __shared__ float red[kNormNT / 64], rss[kNormNT / 64];
+  const int m = blockIdx.x, tid = threadIdx.x, chunks = H >> 3;
+  const bool real = m < T;
+  float v[kNormR][8];
+  float ss = 0.0f, mx = 0.0f;
+#pragma unroll
+  for (int j = 0; j < kNormR; j++) {
+    const int c = tid + kNormNT * j;
+    if (c >= chunks || !real) break;
+    float *xr = x + (size_t)m * H + 8 * c;
+    const float *src = xr;
+    bool in = true;
+    if (ids) {
+      const uint32_t id = ids[m];
+      in = id < (uint32_t)vocab;
+      src = embed + (in ? (size_t)id * H : 0) + 8 * c;
+    }
+    const float4 a = *reinterpret_cast<const float4 *>(src);
+    const float4 b = *reinterpret_cast<const float4 *>(src + 4);
+    const float f[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    float d[8] = {};
+    if (add.p) hrow_get(add, m, 0, c, d);
+    const float4 ga = *reinterpret_cast<const float4 *>(gain + 8 * c);
+    const float4 gb = *reinterpret_cast<const float4 *>(gain + 8 * c + 4);
+    const float g[8] = {ga.x, ga.y, ga.z, ga.w, gb.x, gb.y, gb.z, gb.w};
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      const float s = (in ? f[i] : 0.0f) + d[i];
+      ss += s * s;
+      d[i] = s;
+      v[j][i] = s * g[i];
+      mx = fmaxf(mx, fabsf(v[j][i]));
+    }
+    *reinterpret_cast<float4 *>(xr) = float4{d[0], d[1], d[2], d[3]};
+    *reinterpret_cast<float4 *>(xr + 4) = float4{d[4], d[5], d[6], d[7]};
+  }
+  for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
+  if ((tid & 63) == 0) rss[tid >> 6] = ss;
+  mx = block_max<kNormNT>(mx, red);
+  ss = 0.0f;
+#pragma unroll
+  for (int i = 0; i < kNormNT / 64; i++) ss += rss[i];
+  const float scale = 1.0f / sqrtf(ss / (float)H + eps);
+#pragma unroll
+  for (int j = 0; j < kNormR; j++)
+#pragma unroll
+    for (int i = 0; i < 8; i++) v[j][i] *= scale;
+  put_row<kNormNT>(v, chunks, mx * scale, real, m, xf, rowmul);
+}
+
+// layer.rs:25-42, 609-627 over the prompt: taps oldest to newest, zeros before
+// the first token.  A row's workgroup forms B*x of its taps itself (ck
+// products a channel) rather than in a pass of their own
+__global__ void __launch_bounds__(kNormNT)
+    k_hrows_conv(HRows p, const float *__restrict__ w, const float *__restrict__ bias, int T,
+                 int I, int ck, float *__restrict__ state, f16x8 *__restrict__ xf,
+                 float *__restrict__ rowmul) {
+  __shared__ float red[kNormNT / 64];
+  const int m = blockIdx.x, tid = threadIdx.x, chunks = I >> 3;
+  const bool real = m < T;
+  float v[kNormR][8];
+  float mx = 0.0f;
+#pragma unroll
+  for (int j = 0; j < kNormR; j++) {
+    const int c = tid + kNormNT * j;
+    if (c >= chunks || !real) break;
+    float sum[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) sum[i] = -0.0f;
+    for (int k = 0; k < ck; k++) {
+      const int t = m - (ck - 1) + k;
+      float bx[8] = {};
+      if (t >= 0) {
+        float b[8], xs[8];
+        hrow_get(p, t, 0, c, b);
+        hrow_get(p, t, 2 * I, c, xs);
+#pragma unroll
+        for (int i = 0; i < 8; i++) bx[i] = b[i] * xs[i];
+      }
+#pragma unroll
+      for (int i = 0; i < 8; i++) {
+        const float q = bx[i] * w[(8 * c + i) * ck + k];
+        sum[i] = sum[i] + q;
+        if (m == T - 1) state[(size_t)(8 * c + i) * ck + k] = bx[i];
+      }
+    }
+    float gate[8];
+    hrow_get(p, m, I, c, gate);
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      v[j][i] = gate[i] * (bias ? sum[i] + bias[8 * c + i] : sum[i]);
+      mx = fmaxf(mx, fabsf(v[j][i]));
+    }
+  }
+  mx = block_max<kNormNT>(mx, red);
+  put_row<kNormNT>(v, chunks, mx, real, m, xf, rowmul);
+}
+
+__global__ void __launch_bounds__(kGluNT)
+    k_hrows_swiglu(HRows gu, int T, int F, f16x8 *__restrict__ xf, float *__restrict__ rowmul) {
+  __shared__ float red[kGluNT / 64];
+  __shared__ uint64_t etab[32];
+  const int m = blockIdx.x, tid = threadIdx.x, chunks = F >> 3;
+  const bool real = m < T;
+  if (tid < 32) etab[tid] = syn_exp2_tab[tid];
+  __syncthreads();
+  float v[kGluR][8];
+  float mx = 0.0f;
+#pragma unroll
+  for (int j = 0; j < kGluR; j++) {
+    const int c = tid + kGluNT * j;
+    if (c >= chunks || !real) break;
+    float g[8], u[8];
+    hrow_get(gu, m, 0, c, g);
+    hrow_get(gu, m, F, c, u);
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      v[j][i] = syn_silu_tab(g[i], etab) * u[i];
+      mx = fmaxf(mx, fabsf(v[j][i]));
+    }
+  }
+  mx = block_max<kGluNT>(mx, red);
+  put_row<kGluNT>(v, chunks, mx, real, m, xf, rowmul);
+}
+
+__global__ void __launch_bounds__(256)
+    k_hrows_last(const float *__restrict__ x, HRows add, int T, int H, long long *__restrict__ r) {
+  const int c = blockIdx.x * 256 + threadIdx.x;
+  if (8 * c >= H) return;
+  float d[8];
+  hrow_get(add, T - 1, 0, c, d);
+#pragma unroll
+  for (int i = 0; i < 8; i++) r[8 * c + i] = kqf_fix(x[(size_t)(T - 1) * H + 8 * c + i] + d[i]);
+}
+
+}  // namespace
+
+syn_status_t launch_hrows_norm(float *x, const float *embed, const uint32_t *ids, int vocab,
+                               HRows add, const float *gain, float eps, int T, int H, void *xf,
+                               hipStream_t s) {
+  if (H % 8 || H > kHrowsMaxH) return SYN_ERR_INVALID_ARG;
+  hipLaunchKernelGGL(k_hrows_norm, dim3((unsigned)round_up(T, 32)), dim3(kNormNT), 0, s, x, embed,
+                     ids, vocab, add, gain, eps, T, H, static_cast<f16x8 *>(xf),
+                     rows_frag_scales(xf, T, H, true));
+  SYN_LAUNCH_CHECK();
+  return SYN_OK;
+}
+
+syn_status_t launch_hrows_conv(HRows p, const float *w, const float *bias, int T, int I, int ck,
+                               float *state, void *xf, hipStream_t s) {
+  if (I % 8 || I > kHrowsMaxH) return SYN_ERR_INVALID_ARG;
+  hipLaunchKernelGGL(k_hrows_conv, dim3((unsigned)round_up(T, 32)), dim3(kNormNT), 0, s, p, w,
+                     bias, T, I, ck, state, static_cast<f16x8 *>(xf),
+                     rows_frag_scales(xf, T, I, true));
+  SYN_LAUNCH_CHECK();
+  return SYN_OK;
+}
+
+syn_status_t launch_hrows_swiglu(HRows gu, int T, int F, void *xf, hipStream_t s) {
+  if (F % 8 || F > kHrowsMaxF) return SYN_ERR_INVALID_ARG;
+  hipLaunchKernelGGL(k_hrows_swiglu, dim3((unsigned)round_up(T, 32)), dim3(kGluNT), 0, s, gu, T, F,
+                     static_cast<f16x8 *>(xf), rows_frag_scales(xf, T, F, true));
+  SYN_LAUNCH_CHECK();
+  return SYN_OK;
+}
+
+syn_status_t launch_hrows_last(const float *x, HRows add, int T, int H, long long *r,
+                               hipStream_t s) {
+  if (H % 8) return SYN_ERR_INVALID_ARG;
+  hipLaunchKernelGGL(k_hrows_last, dim3((unsigned)cdiv((size_t)H / 8, 256)), dim3(256), 0, s, x,
+                     add, T, H, r);
+  SYN_LAUNCH_CHECK();
+  return SYN_OK;
+}
+
+}  // namespace syn

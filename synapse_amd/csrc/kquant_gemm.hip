@@ -956,7 +956,7 @@ static syn_status_t kq_gemm_f16(int fmt, bool exact, const u32x4 *W, const uint1
     g.k = k;
     // K splits add into rows that the conversion clears 16 bytes at a time
     const bool can_split = ldy % 4 == 0 && reinterpret_cast<uintptr_t>(d_y) % 16 == 0;
-    const int kz = can_split ? rows_gemm_splits(g, m) : 1;
+    const int kz = can_split ? rows_gemm_splits(g, m, false) : 1;
     SYN_TRY(ensure_rows(f16_rows_bytes(m, k), xh, xh_bytes));
     SYN_TRY(launch_rows_frag(fmt, d_x, ldx, m, k, false, xh.p, kz > 1 ? d_y : nullptr, ldy, n, s));
     return launch_rows_gemm(g, xh.p, m, kz, d_y, ldy, s);

@@ -20,19 +20,19 @@
 #include <algorithm>
 
 #include "kquant.hpp"
+#include "rows_frag.hpp"
 #include "rows_gemm.hpp"
 
 namespace syn {
 
 namespace {
 
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int RW = 8;        // waves per workgroup
 constexpr int RNT = 64 * RW;
-constexpr int KSTEP = 64;
+constexpr int KSTEP = kFragStep;
 
 constexpr bool nibble_order(int fmt) { return fmt != SYN_HIP_FMT_Q8_0; }
 
@@ -335,8 +335,7 @@ __global__ void __launch_bounds__(RNT) __attribute__((amdgpu_waves_per_eu(2, 2))
 }
 
 // One workgroup per row (the padding rows of the last tile are zeros): the
-// row scale that puts the largest magnitude in [2^14, 2^15) (kquant_gemm.hip
-// k_f32_to_f16), then chunk c of eight values to its lane's place.  A row of
+// row scale, then chunk c of eight values to its lane's place.  A row of
 // up to 16384 elements is read once, into registers.
 constexpr int FNT = 512;
 
@@ -386,30 +385,14 @@ __global__ void __launch_bounds__(FNT)
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < FNT / 64; i++) mx = fmaxf(mx, red[i]);
-  float up = 1.0f, down = 1.0f;
-  if (mx > 0.0f && mx <= 3.4028235e38f) {
-    int e;
-    (void)frexpf(mx, &e);
-    e = max(e, 15 - 126);  // a row of subnormals: 2^126 at most
-    up = ldexpf(1.0f, 15 - e);
-    down = ldexpf(1.0f, e - 15);
-  }
+  float up, down;
+  frag_row_scale(mx, &up, &down);
   if (tid == 0) rowmul[m] = down;
-  if (m >= M) up = 0.0f;
   auto put = [&](int c, const float(&v)[8]) {
-    constexpr int ord[8] = {0, 2, 4, 6, 1, 3, 5, 7};
-    f16x8 hi, lo;
+    float t[8];
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-      const float s = m < M ? v[PERM ? ord[i] : i] * up : 0.0f;
-      hi[i] = (_Float16)s;
-      if constexpr (SPLIT) lo[i] = (_Float16)(s - (float)hi[i]);
-    }
-    // chunk c: step c / 8, half (c / 4) % 2, group c % 4
-    const size_t at = (((size_t)(m >> 5) * steps + (c >> 3)) * 4 + (c & 3)) * (SPLIT ? 2 : 1);
-    const int lane = ((c >> 2) & 1) * 32 + (m & 31);
-    xf[at * 64 + lane] = hi;
-    if constexpr (SPLIT) xf[(at + 1) * 64 + lane] = lo;
+    for (int i = 0; i < 8; i++) t[i] = m < M ? v[i] * up : 0.0f;
+    frag_put<PERM, SPLIT>(xf, steps, m, c, t);
   };
 #pragma unroll
   for (int j = 0; j < R; j++)
@@ -423,9 +406,6 @@ __global__ void __launch_bounds__(FNT)
   for (int c = chunks + tid; c < 8 * steps; c += FNT) put(c, zero);
 }
 
-size_t frag_halfs(size_t m, size_t k, bool split) {
-  return round_up(m, 32) * round_up(k, KSTEP) * (split ? 2 : 1);
-}
 
 // Columns per workgroup and K splits (at least two steps per wave) with the
 // least time by this count, in steps of a 32-column wave (~0.8 us each): 256
@@ -462,13 +442,24 @@ Shape shape_of(const RowsGemm &g, size_t m, int kz_max, bool split) {
   return o;
 }
 
+size_t frag_halfs(size_t m, size_t k, bool split) {
+  return round_up(m, 32) * round_up(k, KSTEP) * (split ? 2 : 1);
+}
+
+}  // namespace
+
+float *rows_frag_scales(void *xf, size_t m, size_t k, bool split) {
+  return reinterpret_cast<float *>(static_cast<_Float16 *>(xf) + frag_halfs(m, k, split));
+}
+
+namespace {
+
 template <int FMT, int MT, int NT, bool SPLIT>
 void go(const RowsGemm &g, const Shape &o, const void *xf, size_t m, float *y, size_t ldy,
         size_t zs, hipStream_t s) {
   const dim3 grid((unsigned)cdiv(g.n, (size_t)(32 * NT)), (unsigned)cdiv(m, (size_t)(32 * MT)),
                   (unsigned)o.kz);
-  const float *rowmul = reinterpret_cast<const float *>(
-      static_cast<const _Float16 *>(xf) + frag_halfs(m, g.k, SPLIT));
+  const float *rowmul = rows_frag_scales(const_cast<void *>(xf), m, g.k, SPLIT);
   hipLaunchKernelGGL((k_rows_gemm<FMT, MT, NT, SPLIT>), grid, dim3(RNT), 0, s,
                      static_cast<const u32x4 *>(g.W), g.Wd, (int)g.n, g.blocks,
                      static_cast<const f16x8 *>(xf), rowmul, (int)m, (int)cdiv(g.k, KSTEP), o.per,
@@ -505,7 +496,9 @@ bool rows_gemm_fits(int fmt, bool q8_exact, size_t m, size_t n, size_t k) {
          (m <= 1024 && m * n * k <= 2200000000u);
 }
 
-int rows_gemm_splits(const RowsGemm &g, size_t m) { return shape_of(g, m, kRowsMaxSplit, false).kz; }
+int rows_gemm_splits(const RowsGemm &g, size_t m, bool split) {
+  return shape_of(g, m, kRowsMaxSplit, split).kz;
+}
 
 syn_status_t launch_rows_frag(int fmt, const float *x, size_t ldx, size_t m, size_t k, bool split,
                               void *xf, float *y0, size_t ldy, size_t ny, hipStream_t s) {
@@ -513,7 +506,7 @@ syn_status_t launch_rows_frag(int fmt, const float *x, size_t ldx, size_t m, siz
     set_error("GEMM activation stride must be a multiple of 4 floats and K of 8");
     return SYN_ERR_SHAPE_MISMATCH;
   }
-  float *rowmul = reinterpret_cast<float *>(static_cast<_Float16 *>(xf) + frag_halfs(m, k, split));
+  float *rowmul = rows_frag_scales(xf, m, k, split);
   const auto kern = nibble_order(fmt) ? (split ? k_rows_frag<true, true> : k_rows_frag<true, false>)
                                       : (split ? k_rows_frag<false, true> : k_rows_frag<false, false>);
   hipLaunchKernelGGL(kern, dim3((unsigned)round_up(m, 32)), dim3(FNT), 0, s, x, (int)ldx, (int)m,

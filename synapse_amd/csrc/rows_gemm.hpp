@@ -11,6 +11,8 @@ namespace syn {
 // whole tiles), each row scaled by a power of two, then the rows' inverse
 // scales.  split: each value as the sum of two f16 (22 significant bits).
 size_t rows_frag_bytes(size_t m, size_t k, bool split);
+// the rows' inverse scales inside the buffer
+float *rows_frag_scales(void *xf, size_t m, size_t k, bool split);
 
 struct RowsGemm {
   int fmt = 0;
@@ -27,7 +29,7 @@ syn_status_t launch_rows_frag(int fmt, const float *x, size_t ldx, size_t m, siz
 
 constexpr int kRowsMaxSplit = 8;
 // K splits the launch below would use at best
-int rows_gemm_splits(const RowsGemm &g, size_t m);
+int rows_gemm_splits(const RowsGemm &g, size_t m, bool split);
 // y [m, n] = x W^T from fragments without split, in at most kz K splits (more
 // than one adds into a cleared y).  Weights and activations are rounded once
 // to f16; sums in f32.
