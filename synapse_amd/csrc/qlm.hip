@@ -239,7 +239,7 @@ struct syn_hip_qlm_s {
     SYN_TRY(lm_head.gemv(1, xq.as<int8_t>(), ldh, sx.as<float>(), logits.as<float>(), vocab, s));
     if (sampling)
       return launch_sample(logits.as<float>(), (int)vocab, history.as<uint32_t>(), 0, sargs,
-                           u_draws.as<float>(), st(), add_pos, history.as<uint32_t>(),
+                           u_draws.as<float>(), 0.0f, st(), add_pos, history.as<uint32_t>(),
                            mhist.as<float>(), sscr, nullptr, s);
     SYN_TRY(launch_argmax(logits.as<float>(), (int)vocab, pv.as<float>(), pi.as<int>(),
                           pv2.as<float>(), st(), history.as<uint32_t>(), mhist.as<float>(), s));
@@ -370,7 +370,7 @@ struct syn_hip_qlm_s {
     SYN_TRY(trace_begin(s));
     if (sampling)
       SYN_TRY(launch_sample(logits.as<float>(), (int)vocab, history.as<uint32_t>(), 0, sargs,
-                            u_draws.as<float>(), st(), 1, history.as<uint32_t>(),
+                            u_draws.as<float>(), 0.0f, st(), 1, history.as<uint32_t>(),
                             mhist.as<float>(), sscr, nullptr, s));
     else
       SYN_TRY(launch_argmax_advance(pv.as<float>(), pi.as<int>(), pv2.as<float>(),
