@@ -9,6 +9,7 @@
 // chunk; only the f32 epilogue order is fixed.
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 #include <vector>
 
 #include <mutex>
@@ -19,45 +20,76 @@
 namespace syn {
 
 // --------------------------------------------------------------- quantizer
-// one workgroup per row; max|x| is order-free, the rest is elementwise
-__global__ void __launch_bounds__(256) k_quantize_rows(const float *__restrict__ x, int K,
-                                                       int ldx, int8_t *__restrict__ q, int ldq,
-                                                       float *__restrict__ scales) {
-  __shared__ float red[256];
-  const int row = blockIdx.x;
+// one workgroup per row; max|x| is order-free, the rest is elementwise.  The
+// value's 8-bit level for inv = 127 / max (quantize.zig:12-47)
+__device__ __forceinline__ int8_t q8_level(float v, float inv) {
+  float r = roundf(v * inv);
+  r = fminf(127.0f, fmaxf(-127.0f, r));
+  return (int8_t)(int)r;
+}
+__device__ __forceinline__ uint32_t q8_pack(const float4 &v, float inv) {
+  return (uint32_t)(uint8_t)q8_level(v.x, inv) | (uint32_t)(uint8_t)q8_level(v.y, inv) << 8 |
+         (uint32_t)(uint8_t)q8_level(v.z, inv) << 16 | (uint32_t)(uint8_t)q8_level(v.w, inv) << 24;
+}
+// max|x|, NaN ignored
+__device__ __forceinline__ float amax4(float mx, const float4 &v) {
+  return fmaxf(fmaxf(mx, fmaxf(fabsf(v.x), fabsf(v.y))), fmaxf(fabsf(v.z), fabsf(v.w)));
+}
+
+// VEC: rows of whole 16-byte groups (x, ldx, K and the q rows 4-aligned), up
+// to R of them per thread in registers: one read of the row, all its loads in
+// flight together (512 rows of 4096: 10.0 us with a load per value and pass,
+// 5.0 now; 16 x 14336 with its GEMV 50 against 39)
+template <bool VEC, int R>
+__global__ void __launch_bounds__(256)
+    k_quantize_rows(const float *__restrict__ x, int K, int ldx, int8_t *__restrict__ q, int ldq,
+                    float *__restrict__ scales) {
+  __shared__ float red[4];
+  const int row = blockIdx.x, tid = threadIdx.x;
   const float *xr = x + (size_t)row * ldx;
   int8_t *qr = q + (size_t)row * ldq;
   float mx = 0.0f;
-  for (int j = threadIdx.x; j < K; j += 256) {
-    const float a = fabsf(xr[j]);
-    if (a > mx) mx = a;
+  float4 v[VEC ? R : 1];
+  if constexpr (VEC) {
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+      const int c = tid + 256 * j;
+      v[j] = 4 * c < K ? reinterpret_cast<const float4 *>(xr)[c] : float4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+#pragma unroll
+    for (int j = 0; j < R; j++) mx = amax4(mx, v[j]);
+  } else {
+    for (int j = tid; j < K; j += 256) mx = fmaxf(mx, fabsf(xr[j]));
   }
-  red[threadIdx.x] = mx;
+  for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+  if ((tid & 63) == 0) red[tid >> 6] = mx;
   __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if (threadIdx.x < s) red[threadIdx.x] = fmaxf(red[threadIdx.x], red[threadIdx.x + s]);
-    __syncthreads();
-  }
-  const float max_abs = red[0];
-  if (max_abs == 0.0f) {
-    for (int j = threadIdx.x; j < K; j += 256) qr[j] = 0;
-    if (threadIdx.x == 0) scales[row] = 1.0f;
-    return;
-  }
+  const float max_abs = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+  const bool zero = max_abs == 0.0f;
   const float inv = 127.0f / max_abs;
-  for (int j = threadIdx.x; j < K; j += 256) {
-    float r = roundf(xr[j] * inv);
-    r = fminf(127.0f, fmaxf(-127.0f, r));
-    qr[j] = (int8_t)(int)r;
+  if constexpr (VEC) {
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+      const int c = tid + 256 * j;
+      if (4 * c < K) reinterpret_cast<uint32_t *>(qr)[c] = zero ? 0u : q8_pack(v[j], inv);
+    }
+  } else {
+    for (int j = tid; j < K; j += 256) qr[j] = zero ? (int8_t)0 : q8_level(xr[j], inv);
   }
-  if (threadIdx.x == 0) scales[row] = max_abs / 127.0f;
+  if (tid == 0) scales[row] = zero ? 1.0f : max_abs / 127.0f;
 }
 
 syn_status_t launch_quantize_rows(const float *d_x, size_t m, size_t k, size_t ldx, int8_t *d_q,
                                   size_t ldq, float *d_s, hipStream_t s) {
   if (m == 0 || k == 0) return SYN_OK;
-  hipLaunchKernelGGL(k_quantize_rows, dim3((unsigned)m), dim3(256), 0, s, d_x, (int)k, (int)ldx,
-                     d_q, (int)ldq, d_s);
+  const bool vec = k % 4 == 0 && ldx % 4 == 0 && ldq % 4 == 0 && (uintptr_t)d_x % 16 == 0 &&
+                   (uintptr_t)d_q % 4 == 0 && k <= 16384;
+  const auto kern = !vec         ? k_quantize_rows<false, 1>
+                    : k <= 1024  ? k_quantize_rows<true, 1>
+                    : k <= 4096  ? k_quantize_rows<true, 4>
+                                 : k_quantize_rows<true, 16>;
+  hipLaunchKernelGGL(kern, dim3((unsigned)m), dim3(256), 0, s, d_x, (int)k, (int)ldx, d_q,
+                     (int)ldq, d_s);
   SYN_LAUNCH_CHECK();
   return SYN_OK;
 }
@@ -159,6 +191,82 @@ __global__ void __launch_bounds__(1024)
     } else {
       part[((size_t)ks * M + m) * N64 + row] = s;
     }
+  }
+}
+
+// The same GEMV from one f32 row: every workgroup forms the row's maximum (all
+// of K, from L2) and quantizes its own K slice into LDS, with its first
+// weights already requested; the quantizer's launch and the round trip
+// between the two kernels are gone (whole calls, us: 1024 -> 1024 7.1 to 4.2,
+// 4096 -> 4096 10.7 to 6.5, 14336 -> 4096 25.4 to 12.5).  Same values:
+// q8_level of the same maximum.
+template <bool SK>
+__global__ void __launch_bounds__(1024)
+    k_gemv_w8a8_x(const i32x4 *__restrict__ W, const float *__restrict__ ws,
+                  const float *__restrict__ x, int K, float *__restrict__ y,
+                  unsigned long long *__restrict__ acc64, int N, int C, int cs) {
+  extern __shared__ __align__(16) int gx_lds[];  // quantized slice [4 cs] | sums [waves][64]
+  __shared__ float rmax[16];
+  const int panel = blockIdx.x, ks = blockIdx.y, tid = threadIdx.x;
+  const int nt = blockDim.x, nw = nt >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int c0 = ks * cs, c1 = min(C, c0 + cs);
+  int *xq = gx_lds, *red = gx_lds + 4 * cs;
+  const i32x4 *Wp = W + (size_t)panel * C * 64 + lane;
+  // the wave's first two chunks (clamped; used if they are its own)
+  i32x4 wp[2];
+#pragma unroll
+  for (int u = 0; u < 2; u++)
+    wp[u] = __builtin_nontemporal_load(Wp + (size_t)min(c0 + wave + u * nw, c1 - 1) * 64);
+  const float4 *x4 = reinterpret_cast<const float4 *>(x);
+  float mx = 0.0f;
+#pragma unroll 4
+  for (int c = tid; c < K >> 2; c += nt) mx = amax4(mx, x4[c]);
+  for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+  if (lane == 0) rmax[wave] = mx;
+  __syncthreads();
+  for (int w = 0; w < nw; w++) mx = fmaxf(mx, rmax[w]);
+  const float inv = 127.0f / mx;
+  for (int j = tid; j < 4 * (c1 - c0); j += nt) {  // groups of four values; past K zeros
+    const int k4 = 4 * c0 + j;
+    const float4 v = x4[min(k4, (K >> 2) - 1)];
+    xq[j] = 4 * k4 < K && mx != 0.0f ? (int)q8_pack(v, inv) : 0;
+  }
+  __syncthreads();
+  int acc = 0;
+  auto dot = [&](const i32x4 &w, int c) {
+    const i32x4 xv = *reinterpret_cast<const i32x4 *>(xq + 4 * (c - c0));
+    acc = __builtin_amdgcn_sdot4(w.x, xv.x, acc, false);
+    acc = __builtin_amdgcn_sdot4(w.y, xv.y, acc, false);
+    acc = __builtin_amdgcn_sdot4(w.z, xv.z, acc, false);
+    acc = __builtin_amdgcn_sdot4(w.w, xv.w, acc, false);
+  };
+#pragma unroll
+  for (int u = 0; u < 2; u++)
+    if (c0 + wave + u * nw < c1) dot(wp[u], c0 + wave + u * nw);
+#pragma unroll 4
+  for (int c = c0 + wave + 2 * nw; c < c1; c += nw)
+    dot(__builtin_nontemporal_load(Wp + (size_t)c * 64), c);
+  red[wave * 64 + lane] = acc;
+  __syncthreads();
+  if (tid >= 64) return;
+  const int row = panel * 64 + tid;
+  const float sx = mx == 0.0f ? 1.0f : mx / 127.0f;
+  int s = 0;
+  for (int w = 0; w < nw; w++) s += red[w * 64 + tid];
+  if constexpr (SK) {  // as in k_gemv_w8a8
+    unsigned long long *a = acc64 + row;
+    const unsigned long long add = (1ull << 40) + (unsigned long long)(long long)s;
+    const unsigned long long tot =
+        __hip_atomic_fetch_add(a, add, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + add;
+    const long long sum = (long long)(tot << 24) >> 24;
+    if ((int)((tot - (unsigned long long)sum) >> 40) != (int)gridDim.y) return;
+    __hip_atomic_store(a, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    s = (int)sum;
+  }
+  if (row < N) {
+    const float f = (float)s * sx;
+    y[row] = f * ws[row];
   }
 }
 
@@ -275,6 +383,29 @@ syn_status_t QLinearInt8::gemv(size_t m, const int8_t *d_xq, size_t ldx, const f
   const GemvPlan p = make_gemv_plan(n, (size_t)chunks, false);
   kGemvLaunch[m](p, w.as<i32x4>(), scales.as<float>(), d_xq, (int)ldx, d_sx, d_y, (int)ldy,
                  nullptr, sk_acc.as<unsigned long long>(), (int)n, s);
+  SYN_LAUNCH_CHECK();
+  return SYN_OK;
+}
+
+// Whether a forward quantizes inside the GEMV: one row, on grids of up to two
+// workgroups per CU (each repeats the maximum: 1024 -> 32768, 512 workgroups,
+// 9.2 to 7.2 us; a vocabulary's 2374 would repeat it nine times over).  Two
+// rows double that work: 4096 -> 4096 8.5 us against 8.4 in two launches.
+bool QLinearInt8::forward_fits(size_t m, const float *d_x) const {
+  if (m != 1 || n == 0 || k == 0 || k % 4 || k > 16384 || (uintptr_t)d_x % 16) return false;
+  const GemvPlan p = make_gemv_plan(n, (size_t)chunks, false);
+  return p.panels * p.ksplit <= 512;
+}
+
+syn_status_t QLinearInt8::forward_f32(const float *d_x, float *d_y, hipStream_t s) {
+  SYN_TRY(ensure_sk());
+  const GemvPlan p = make_gemv_plan(n, (size_t)chunks, false);
+  const int waves = std::max(4, p.waves);  // at least 256 threads share the row's maximum
+  const size_t shm = (4 * (size_t)p.cs + (size_t)waves * 64) * sizeof(int);
+  const auto kern = p.ksplit > 1 ? k_gemv_w8a8_x<true> : k_gemv_w8a8_x<false>;
+  hipLaunchKernelGGL(kern, dim3(p.panels, p.ksplit), dim3(64 * waves), shm, s, w.as<i32x4>(),
+                     scales.as<float>(), d_x, (int)k, d_y, sk_acc.as<unsigned long long>(), (int)n,
+                     p.chunks, p.cs);
   SYN_LAUNCH_CHECK();
   return SYN_OK;
 }
@@ -520,6 +651,7 @@ syn_status_t syn_hip_qlinear_forward(syn_hip_qlinear_t *h, size_t m, const float
   if (h->fmt == SYN_HIP_FMT_TERNARY) return h->ter.gemv(m, d_x, h->ter.k, d_y, h->ter.n, s);
   if (h->fmt != SYN_HIP_FMT_INT8) return SYN_ERR_INVALID_ARG;
   QLinearInt8 &L = h->i8;
+  if (L.forward_fits(m, d_x)) return L.forward_f32(d_x, d_y, s);
   const size_t ldq = (size_t)L.chunks * 16;
   if (L.xq_rows < m) {
     SYN_HIP(hipDeviceSynchronize());

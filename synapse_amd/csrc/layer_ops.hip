@@ -905,7 +905,9 @@ syn_status_t launch_attention_prefill(const float *q, const float *kcache, const
 }
 
 // ------------------------------------------------------------------ SwiGLU + quantize
-__global__ void __launch_bounds__(256)
+// one workgroup per row; a wide row takes 1024 threads (128 rows of 3072: 13.1
+// us with 256, 6.4 with 1024)
+__global__ void __launch_bounds__(1024)
     k_swiglu_quant(const float *__restrict__ gu, int ldgu, int inter, int8_t *__restrict__ hq,
                    int ldq, float *__restrict__ sh) {
   extern __shared__ float sm[];  // inter
@@ -922,8 +924,8 @@ __global__ void __launch_bounds__(256)
 
 syn_status_t launch_swiglu_quant(const float *gu, int ldgu, int rows, int inter, int8_t *hq,
                                  int ldq, float *sh, hipStream_t s) {
-  hipLaunchKernelGGL(k_swiglu_quant, dim3(rows), dim3(256), inter * sizeof(float), s, gu, ldgu,
-                     inter, hq, ldq, sh);
+  hipLaunchKernelGGL(k_swiglu_quant, dim3(rows), dim3(inter >= 1024 ? 1024 : 256),
+                     inter * sizeof(float), s, gu, ldgu, inter, hq, ldq, sh);
   SYN_LAUNCH_CHECK();
   return SYN_OK;
 }

@@ -61,6 +61,9 @@ struct QLinearInt8 {
   syn_status_t gemv_part(size_t m, const int8_t *d_xq, size_t ldx, const float *d_sx,
                          float *d_y, size_t ldy, int *d_part, hipStream_t s);
   size_t part_elems_for(size_t m) const;
+  // y = forward of one f32 row in one launch, quantized inside
+  bool forward_fits(size_t m, const float *d_x) const;
+  syn_status_t forward_f32(const float *d_x, float *d_y, hipStream_t s);
   syn_status_t ensure_part(size_t elems);
   // allocate split-K scratch for up to max_m activation rows (needed before
   // a graph capture: nothing may allocate while a step is being recorded)
