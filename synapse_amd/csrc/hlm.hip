@@ -237,6 +237,7 @@ struct syn_hip_hlm_s {
   DevBuf x, normed, proj, conv_out, qrot, attn, o, gu, hbuf, down, logits;
   DevBuf state, pv, pi, pv2, history, mhist;
   hipStream_t stream = nullptr;
+  HostPos hp;
   hipGraphExec_t graph = nullptr;
   bool ready = false, use_graph = true;
   // fused step (klm_fused.hip's GEMV over the Q4_0 planes): the fixed-point
@@ -558,20 +559,30 @@ struct syn_hip_hlm_s {
     return SYN_OK;
   }
   syn_status_t run_step() {
+    hp.known = false;
     if (!use_graph) return decode_step(stream);
     SYN_TRY(build_graph());
     SYN_HIP(hipGraphLaunch(graph, stream));
     return SYN_OK;
   }
-  syn_status_t set_state(int pos, uint32_t token, int step) {
-    StepState hs{pos, token, step, 0.0f};
-    SYN_HIP(hipMemcpyAsync(state.p, &hs, sizeof(hs), hipMemcpyHostToDevice, stream));
-    SYN_HIP(hipStreamSynchronize(stream));
-    return SYN_OK;
+  syn_status_t set_state(int pos, uint32_t token, int step_) {
+    hp.known = false;
+    return launch_state_init(st(), pos, token, step_, stream);
   }
   syn_status_t get_state(StepState *out) {
     SYN_HIP(hipMemcpyAsync(out, state.p, sizeof(StepState), hipMemcpyDeviceToHost, stream));
     SYN_HIP(hipStreamSynchronize(stream));
+    return SYN_OK;
+  }
+  // position and step of the device state: known, or read back
+  syn_status_t where(int *pos, int *step) {
+    if (!hp.known) {
+      StepState cur;
+      SYN_TRY(get_state(&cur));
+      hp = HostPos{true, cur.pos, cur.step};
+    }
+    *pos = hp.pos;
+    *step = hp.step;
     return SYN_OK;
   }
   // conv states to zero, position 0 (the KV rows past the position are never read)
@@ -774,17 +785,18 @@ syn_status_t syn_hip_hlm_position(syn_hip_hlm_t *m, size_t *pos) {
 
 syn_status_t syn_hip_hlm_decode_one(syn_hip_hlm_t *m, uint32_t token, float *host_logits) {
   SYN_TRY(check_hlm(m));
-  StepState cur;
-  SYN_TRY(m->get_state(&cur));
-  if ((size_t)cur.pos >= m->S) {
+  int pos, step;
+  SYN_TRY(m->where(&pos, &step));
+  if ((size_t)pos >= m->S) {
     set_error("hybrid LM: KV cache full");
     return SYN_ERR_INVALID_ARG;
   }
-  SYN_TRY(m->set_state(cur.pos, token, cur.step));
+  SYN_TRY(m->set_state(pos, token, step));
   SYN_TRY(m->run_step());
   if (host_logits)
     SYN_HIP(hipMemcpyAsync(host_logits, m->logits.p, m->V * 4, hipMemcpyDeviceToHost, m->stream));
   SYN_HIP(hipStreamSynchronize(m->stream));
+  m->hp = HostPos{true, pos + 1, step + 1};
   return SYN_OK;
 }
 
@@ -793,20 +805,21 @@ syn_status_t syn_hip_hlm_prefill(syn_hip_hlm_t *m, const uint32_t *ids, size_t n
   SYN_TRY(check_hlm(m));
   if (!ids) return SYN_ERR_NULL_PTR;
   if (n == 0) return SYN_OK;
-  StepState cur;
-  SYN_TRY(m->get_state(&cur));
+  int pos, step;
+  SYN_TRY(m->where(&pos, &step));
   size_t i = 0;
   // into an empty cache all at once (the rest of a longer prompt, and a
   // prompt into a filled cache, token by token)
-  if (cur.pos == 0 && n >= m->kRowsMin && n <= m->S && m->rows_supported()) {
+  if (pos == 0 && n >= m->kRowsMin && n <= m->S && m->rows_supported()) {
     i = std::min(n, m->kRowsMax);
-    SYN_TRY(m->prefill_rows(ids, i, cur.step + (int)i - 1));
+    SYN_TRY(m->prefill_rows(ids, i, step + (int)i - 1));
     if (i == n) {
       if (host_logits)
         SYN_HIP(hipMemcpyAsync(host_logits, m->logits.p, m->V * 4, hipMemcpyDeviceToHost,
                                m->stream));
       SYN_HIP(hipStreamSynchronize(m->stream));
     }
+    m->hp = HostPos{true, (int)i, step + (int)i};
   }
   for (; i < n; i++)
     SYN_TRY(syn_hip_hlm_decode_one(m, ids[i], i + 1 == n ? host_logits : nullptr));

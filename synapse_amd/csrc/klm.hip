@@ -36,6 +36,7 @@ struct syn_hip_klm_s {
   DevBuf x, normed, qkv, qrot, attn, o, gu, hbuf, down, logits, scores;
   DevBuf pv, pi, pv2, state, history, mhist, ids;
   hipStream_t stream = nullptr;
+  HostPos hp;
   hipGraphExec_t graph = nullptr;
   bool finalized = false;
   bool use_graph = true;  // replay the captured decode step, else launch eagerly
@@ -353,22 +354,32 @@ struct syn_hip_klm_s {
 
   // one decode step on `stream`: graph replay or the same kernels launched eagerly
   syn_status_t run_step() {
+    hp.known = false;
     if (!use_graph) return decode_step(stream);
     SYN_TRY(build_graph());
     SYN_HIP(hipGraphLaunch(graph, stream));
     return SYN_OK;
   }
 
-  syn_status_t set_state(int pos, uint32_t token, int step) {
-    StepState hs{pos, token, step, 0.0f};
-    SYN_HIP(hipMemcpyAsync(state.p, &hs, sizeof(hs), hipMemcpyHostToDevice, stream));
-    SYN_HIP(hipStreamSynchronize(stream));
-    return SYN_OK;
+  syn_status_t set_state(int pos, uint32_t token, int step_) {
+    hp.known = false;
+    return launch_state_init(st(), pos, token, step_, stream);
   }
 
   syn_status_t get_state(StepState *out) {
     SYN_HIP(hipMemcpyAsync(out, state.p, sizeof(StepState), hipMemcpyDeviceToHost, stream));
     SYN_HIP(hipStreamSynchronize(stream));
+    return SYN_OK;
+  }
+  // position and step of the device state: known, or read back
+  syn_status_t where(int *pos, int *step) {
+    if (!hp.known) {
+      StepState cur;
+      SYN_TRY(get_state(&cur));
+      hp = HostPos{true, cur.pos, cur.step};
+    }
+    *pos = hp.pos;
+    *step = hp.step;
     return SYN_OK;
   }
 
@@ -401,6 +412,7 @@ struct syn_hip_klm_s {
       set_error("prefill rows must be in [1, max_seq - cached rows]");
       return SYN_ERR_INVALID_ARG;
     }
+    hp.known = false;
     SYN_HIP(hipMemcpyAsync(ids.p, host_ids, n * 4, hipMemcpyHostToDevice, stream));
     SYN_TRY(prefill_rows(ids.as<uint32_t>(), (int)n, cur.pos));
     return head((int)n - 1, (int)n, stream);
@@ -638,6 +650,7 @@ syn_status_t syn_hip_klm_forward_prefill(syn_hip_klm_t *m, const uint32_t *ids, 
     SYN_HIP(hipMemcpyAsync(host_logits, m->logits.p, m->vocab * 4, hipMemcpyDeviceToHost,
                            m->stream));
   SYN_HIP(hipStreamSynchronize(m->stream));
+  m->hp = HostPos{true, (int)n, 1};
   return SYN_OK;
 }
 
@@ -670,18 +683,19 @@ syn_status_t syn_hip_klm_cache_len(syn_hip_klm_t *m, size_t *out_len) {
 syn_status_t syn_hip_klm_forward_one_draft(syn_hip_klm_t *m, uint32_t token, size_t n_layers,
                                            float *host_logits) {
   SYN_TRY(check_klm(m));
-  StepState cur;
-  SYN_TRY(m->get_state(&cur));
-  if ((size_t)cur.pos >= m->S) {
+  int pos, step;
+  SYN_TRY(m->where(&pos, &step));
+  if ((size_t)pos >= m->S) {
     set_error("KV cache full");
     return SYN_ERR_INVALID_ARG;
   }
-  SYN_TRY(m->set_state(cur.pos, token, cur.step));
+  SYN_TRY(m->set_state(pos, token, step));
   SYN_TRY(m->run_draft(n_layers));
   if (host_logits)
     SYN_HIP(hipMemcpyAsync(host_logits, m->logits.p, m->vocab * 4, hipMemcpyDeviceToHost,
                            m->stream));
   SYN_HIP(hipStreamSynchronize(m->stream));
+  m->hp = HostPos{true, pos + 1, step + 1};
   return SYN_OK;
 }
 
@@ -707,18 +721,19 @@ syn_status_t syn_hip_klm_generate_speculative(syn_hip_klm_t *m, const uint32_t *
 
 syn_status_t syn_hip_klm_forward_one(syn_hip_klm_t *m, uint32_t token, float *host_logits) {
   SYN_TRY(check_klm(m));
-  StepState cur;
-  SYN_TRY(m->get_state(&cur));
-  if ((size_t)cur.pos >= m->S) {
+  int pos, step;
+  SYN_TRY(m->where(&pos, &step));
+  if ((size_t)pos >= m->S) {
     set_error("KV cache full");
     return SYN_ERR_INVALID_ARG;
   }
-  SYN_TRY(m->set_state(cur.pos, token, cur.step));
+  SYN_TRY(m->set_state(pos, token, step));
   SYN_TRY(m->run_step());
   if (host_logits)
     SYN_HIP(hipMemcpyAsync(host_logits, m->logits.p, m->vocab * 4, hipMemcpyDeviceToHost,
                            m->stream));
   SYN_HIP(hipStreamSynchronize(m->stream));
+  m->hp = HostPos{true, pos + 1, step + 1};
   return SYN_OK;
 }
 

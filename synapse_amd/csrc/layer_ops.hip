@@ -1079,6 +1079,18 @@ syn_status_t launch_kv_zero_rows(float *kc, float *vc, size_t k_stride, size_t v
   return SYN_OK;
 }
 
+__global__ void k_state_init(StepState *st, StepState v) {
+  if (threadIdx.x == 0) *st = v;
+}
+
+syn_status_t launch_state_init(StepState *state, int pos, uint32_t token, int step,
+                               hipStream_t s) {
+  hipLaunchKernelGGL(k_state_init, dim3(1), dim3(64), 0, s, state,
+                     StepState{pos, token, step, 0.0f});
+  SYN_LAUNCH_CHECK();
+  return SYN_OK;
+}
+
 __global__ void k_state_set(StepState *st, int pos, int nhist) {
   if (threadIdx.x == 0) {
     if (pos >= 0) st->pos = pos;

@@ -89,6 +89,17 @@ syn_status_t launch_step_advance(StepState *state, int add_pos, hipStream_t s);
 syn_status_t launch_kv_zero_rows(float *kc, float *vc, size_t k_stride, size_t v_stride,
                                  int layers, int nkv, int hd, int max_seq, const StepState *st,
                                  hipStream_t s);
+// What the host knows of a decoder's StepState.  A call that ends at a known
+// position leaves it here, so that the next step need not read the state back
+// first (a copy and a wait, ~20 us); whatever else changes the state clears
+// `known`.
+struct HostPos {
+  bool known = false;
+  int pos = 0, step = 0;
+};
+// *state = {pos, token, step, 0, all of the history}: by kernel argument, no
+// copy from host memory to wait for
+syn_status_t launch_state_init(StepState *state, int pos, uint32_t token, int step, hipStream_t s);
 // state->pos = pos (if pos >= 0), state->nhist = nhist
 syn_status_t launch_state_set(StepState *state, int pos, int nhist, hipStream_t s);
 // elementwise residual: x += d

@@ -478,6 +478,7 @@ struct syn_hip_mamba_s {
   size_t acc_elems = 0;
   size_t hist_cap = 0;
   hipStream_t stream = nullptr;
+  HostPos hp;
   hipGraphExec_t graph = nullptr;
   bool use_graph = true;  // replay the captured step, else launch eagerly
   bool fused = false;     // fused split-K GEMV step (when the shapes fit)
@@ -737,6 +738,7 @@ struct syn_hip_mamba_s {
 
   // one token step on `stream`: graph replay or the same kernels launched eagerly
   syn_status_t run_step() {
+    hp.known = false;
     if (!use_graph) return step(stream);
     SYN_TRY(build_graph());
     SYN_HIP(hipGraphLaunch(graph, stream));
@@ -744,9 +746,24 @@ struct syn_hip_mamba_s {
   }
 
   syn_status_t set_state(int pos, uint32_t token, int step_) {
-    StepState hs{pos, token, step_, 0.0f};
-    SYN_HIP(hipMemcpyAsync(state.p, &hs, sizeof(hs), hipMemcpyHostToDevice, stream));
+    hp.known = false;
+    return launch_state_init(st(), pos, token, step_, stream);
+  }
+
+  syn_status_t get_state(StepState *out) {
+    SYN_HIP(hipMemcpyAsync(out, state.p, sizeof(StepState), hipMemcpyDeviceToHost, stream));
     SYN_HIP(hipStreamSynchronize(stream));
+    return SYN_OK;
+  }
+  // position and step of the device state: known, or read back
+  syn_status_t where(int *pos, int *step) {
+    if (!hp.known) {
+      StepState cur;
+      SYN_TRY(get_state(&cur));
+      hp = HostPos{true, cur.pos, cur.step};
+    }
+    *pos = hp.pos;
+    *step = hp.step;
     return SYN_OK;
   }
 
@@ -1043,24 +1060,25 @@ syn_status_t syn_hip_mamba_prefill(syn_hip_mamba_t *m, const uint32_t *ids, size
     SYN_HIP(hipMemcpyAsync(host_logits, m->logits.p, m->vocab * 4, hipMemcpyDeviceToHost,
                            m->stream));
   SYN_HIP(hipStreamSynchronize(m->stream));
+  m->hp = HostPos{true, (int)n, 1};
   return SYN_OK;
 }
 
 syn_status_t syn_hip_mamba_decode_one(syn_hip_mamba_t *m, uint32_t token, float *host_logits) {
   SYN_TRY(check_mamba(m));
-  StepState cur;
-  SYN_HIP(hipMemcpyAsync(&cur, m->state.p, sizeof(cur), hipMemcpyDeviceToHost, m->stream));
-  SYN_HIP(hipStreamSynchronize(m->stream));
-  if ((size_t)cur.step + 1 >= m->hist_cap) {
+  int pos, step;
+  SYN_TRY(m->where(&pos, &step));
+  if ((size_t)step + 1 >= m->hist_cap) {
     set_error("max_tokens reached");
     return SYN_ERR_INVALID_ARG;
   }
-  SYN_TRY(m->set_state(cur.pos, token, cur.step));
+  SYN_TRY(m->set_state(pos, token, step));
   SYN_TRY(m->run_step());
   if (host_logits)
     SYN_HIP(hipMemcpyAsync(host_logits, m->logits.p, m->vocab * 4, hipMemcpyDeviceToHost,
                            m->stream));
   SYN_HIP(hipStreamSynchronize(m->stream));
+  m->hp = HostPos{true, pos + 1, step + 1};
   return SYN_OK;
 }
 

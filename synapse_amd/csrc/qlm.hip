@@ -57,6 +57,7 @@ struct syn_hip_qlm_s {
   DevBuf xin, xmid, scal, acc;
   size_t acc_elems = 0;
   hipStream_t stream = nullptr;
+  HostPos hp;
   hipGraphExec_t graph = nullptr;
   bool finalized = false;
   // per-launch event pairs of an eager fused step (syn_hip_qlm_time_step_kernels)
@@ -407,6 +408,7 @@ struct syn_hip_qlm_s {
 
   // one decode step on the model stream: graph replay or eager launches
   syn_status_t run_step() {
+    hp.known = false;
     if (!use_graph) return decode_step(stream);
     SYN_TRY(build_graph());
     SYN_HIP(hipGraphLaunch(graph, stream));
@@ -449,17 +451,25 @@ struct syn_hip_qlm_s {
     return SYN_OK;
   }
 
-  syn_status_t set_state(int pos, uint32_t token, int step) {
-    StepState hs{pos, token, step, 0.0f};
-    // synchronous: hs lives on this stack frame
-    SYN_HIP(hipMemcpyAsync(state.p, &hs, sizeof(hs), hipMemcpyHostToDevice, stream));
-    SYN_HIP(hipStreamSynchronize(stream));
-    return SYN_OK;
+  syn_status_t set_state(int pos, uint32_t token, int step_) {
+    hp.known = false;
+    return launch_state_init(st(), pos, token, step_, stream);
   }
 
   syn_status_t get_state(StepState *out) {
     SYN_HIP(hipMemcpyAsync(out, state.p, sizeof(StepState), hipMemcpyDeviceToHost, stream));
     SYN_HIP(hipStreamSynchronize(stream));
+    return SYN_OK;
+  }
+  // position and step of the device state: known, or read back
+  syn_status_t where(int *pos, int *step) {
+    if (!hp.known) {
+      StepState cur;
+      SYN_TRY(get_state(&cur));
+      hp = HostPos{true, cur.pos, cur.step};
+    }
+    *pos = hp.pos;
+    *step = hp.step;
     return SYN_OK;
   }
 
@@ -493,6 +503,7 @@ struct syn_hip_qlm_s {
       set_error("prefill rows must be in [1, max_seq - cached rows]");
       return SYN_ERR_INVALID_ARG;
     }
+    hp.known = false;
     SYN_HIP(hipMemcpyAsync(ids.p, host_ids, n * 4, hipMemcpyHostToDevice, stream));
     SYN_TRY(prefill_rows(ids.as<uint32_t>(), (int)n, cur.pos));
     return head((int)n - 1, (int)n, stream);
@@ -879,6 +890,7 @@ syn_status_t syn_hip_qlm_forward_prefill(syn_hip_qlm_t *m, const uint32_t *ids, 
     SYN_HIP(hipMemcpyAsync(host_logits, m->logits.p, m->vocab * 4, hipMemcpyDeviceToHost,
                            m->stream));
   SYN_HIP(hipStreamSynchronize(m->stream));
+  m->hp = HostPos{true, (int)n, 1};
   return SYN_OK;
 }
 
@@ -910,19 +922,20 @@ syn_status_t syn_hip_qlm_cache_len(syn_hip_qlm_t *m, size_t *out_len) {
 
 syn_status_t syn_hip_qlm_forward_one(syn_hip_qlm_t *m, uint32_t token, float *host_logits) {
   SYN_TRY(check_model(m));
-  StepState cur;
-  SYN_TRY(m->get_state(&cur));
-  if ((size_t)cur.pos >= m->S) {
+  int pos, step;
+  SYN_TRY(m->where(&pos, &step));
+  if ((size_t)pos >= m->S) {
     set_error("KV cache full");  // kvcache.zig:68-69 CacheFull
     return SYN_ERR_INVALID_ARG;
   }
   if (m->use_graph) SYN_TRY(m->build_graph());
-  SYN_TRY(m->set_state(cur.pos, token, cur.step));
+  SYN_TRY(m->set_state(pos, token, step));
   SYN_TRY(m->run_step());
   if (host_logits)
     SYN_HIP(hipMemcpyAsync(host_logits, m->logits.p, m->vocab * 4, hipMemcpyDeviceToHost,
                            m->stream));
   SYN_HIP(hipStreamSynchronize(m->stream));
+  m->hp = HostPos{true, pos + 1, step + 1};
   return SYN_OK;
 }
 
@@ -1053,6 +1066,7 @@ syn_status_t syn_hip_qlm_time_step_kernels(syn_hip_qlm_t *m, size_t steps, float
   std::vector<syn_hip_qlm_s::TraceEntry> tr;
   tr.reserve(steps * (5 * m->L + 4));
   m->trace = &tr;
+  m->hp.known = false;
   syn_status_t st = SYN_OK;
   for (size_t i = 0; i < steps && st == SYN_OK; i++) st = m->decode_step(m->stream);
   m->trace = nullptr;
