@@ -179,6 +179,33 @@ __device__ __forceinline__ float syn_expf_tab(float x, const uint64_t *tab) {
   return (float)y;
 }
 
+// the same value without a branch (the special cases selected at the end), so
+// that several can be in flight: a branch each keeps them apart
+__device__ __forceinline__ float syn_expf_sel(float x, const uint64_t *tab) {
+  const double InvLn2N = 0x1.71547652b82fep+0 * 32.0;
+  const double SHIFT = 0x1.8p+52;
+  const double C0 = 0x1.c6af84b912394p-5 / 32 / 32 / 32;
+  const double C1 = 0x1.ebfce50fac4f3p-3 / 32 / 32;
+  const double C2 = 0x1.62e42ff0c52d6p-1 / 32;
+  const double xd = (double)x;
+  double kd = __builtin_fma(InvLn2N, xd, SHIFT);
+  const uint64_t ki = (uint64_t)__double_as_longlong(kd);
+  kd -= SHIFT;
+  const double r = __builtin_fma(InvLn2N, xd, -kd);
+  uint64_t t = tab[ki & 31u];
+  t += ki << 47;
+  const double s = __longlong_as_double((long long)t);
+  const double z = __builtin_fma(C0, r, C1);
+  const double r2 = r * r;
+  double y = __builtin_fma(C2, r, 1.0);
+  y = __builtin_fma(z, r2, y);
+  y = y * s;
+  float f = (float)y;
+  f = x > 0x1.62e42ep6f ? __uint_as_float(0x7f800000u) : f;
+  f = x < -0x1.9fe368p6f ? 0.0f : f;
+  return x != x ? x + x : f;
+}
+
 __device__ __forceinline__ float syn_expf(float x) { return syn_expf_tab(x, syn_exp2_tab); }
 
 // reference SiLU: x / (1 + exp(-x))  (ops/activation.rs:30-32)

@@ -430,415 +430,339 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-// Row-block form of k_attn_prefill: one workgroup per (head, 16 query rows),
-// the head's K and V rows staged through LDS 64 positions at a time, so each
-// row of the cache is read once per 16 queries instead of once per query.
-// Every score, sum and product is the one k_attn_prefill forms, in the same
-// order (the same chains per (row, position) and (row, column)).
-constexpr int kPfRows = 16, kPfChunk = 64;
+// Prefill attention on the matrix cores: one workgroup per (head, 16 query
+// rows).  v_mfma_f32_16x16x4_f32 forms each element as four f32 fused
+// multiply-adds in ascending k (checked bit for bit on gfx950 over 2M random
+// elements with cancellation, subnormal sums, infinities and NaN), which is
+// the chain of @mulAdd the reference's full micro-tiles run, so EXACT holds
+// every bit of k_attn_prefill; the few rows and columns that the reference
+// computes as plain a*b + c (its partial micro-tiles) are formed again that
+// way by the vector units.
+//   scores: a wave takes 16 positions; lane (g, m) = (lane / 16, lane % 16)
+//     holds q[row m][4i + g] and k[position m][4i + g] for k-step i; K goes
+//     from memory to registers, no staging.
+//   softmax: 32 threads a row.  EXACT: the online sum's exponentials in
+//     segments of 256 positions (run maxima by a scan), then the dependent
+//     chain on one thread a row; masked positions add nothing to it.  Else max
+//     and sum by shuffles.
+//   P V: a wave takes 16 columns, k-steps run over the positions in order.  A
+//     step's positions outside the block's range count as 0 * -0, the one
+//     product that changes no sum's bits.  EXACT runs over the masked positions
+//     too (0 * v is not always without effect).
+// Both K and V are read 16 bytes a lane and brought into the lanes' layout by
+// a transpose between the four 16-lane groups (4-byte loads in that layout
+// took 4 cycles a 64-byte line each: 16 heads of 128, 128 tokens, 18 us
+// against 13).
+// What bounds it at short prompts is latency (loads, the softmax chain), at
+// long ones reads of K and V, once per 16 rows.  Against VALU kernels that
+// staged K and V through LDS (four or eight FMA for two to nine LDS reads):
+// INT8 decoder, 16 heads of 128, 128 tokens 70.2 -> 12.9 us; tolerance form,
+// 24 heads of 128, 256 tokens 76.1 -> 15.8 us.
+constexpr int kPfRows = 16, kPfThreads = 512, kPfSeg = 256, kPfSegLd = kPfSeg + 4;
 
-template <int HD>
-__global__ void __launch_bounds__(256)
-    k_attn_prefill_rows(const float *__restrict__ q, const float *__restrict__ kc,
+// stride of a row of scores: room for a start at any position of a group of
+// four; 4 mod 64 puts a step's 16 rows x 4 positions in 64 different banks
+__host__ __device__ __forceinline__ int pf_ld(int t) {
+  const int w = (t + 6) & ~3;
+  return (w + 59) / 64 * 64 + 4;
+}
+
+// 4 x 4 transpose between the four groups of 16 lanes and the elements of v:
+// element g of group s goes to element s of group g
+__device__ __forceinline__ f32x4 groups_transposed(f32x4 v) {
+  const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v.x), __float_as_uint(v.z),
+                                                  false, false);
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v.y), __float_as_uint(v.w),
+                                                  false, false);
+  const auto c = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);
+  const auto d = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+  return f32x4{__uint_as_float(c[0]), __uint_as_float(c[1]), __uint_as_float(d[0]),
+               __uint_as_float(d[1])};
+}
+
+template <int HD, bool EXACT>
+__global__ void __launch_bounds__(kPfThreads)
+    k_attn_prefill_mfma(const float *__restrict__ q, const float *__restrict__ kc,
                         const float *__restrict__ vc, int t, int nh, int nkv, int max_seq,
                         int cache_off, float *__restrict__ out) {
-  constexpr int hd = HD;  // compile-time: LDS offsets become immediates
-  extern __shared__ float sm[];
-  // qs[16][hd] | kv[64][hd + 1] | e[16][t] | c[16][t]
-  const int ldk = hd + 1;
-  float *qs = sm, *kv = qs + kPfRows * hd, *e = kv + kPfChunk * ldk, *cj = e + kPfRows * t;
-  __shared__ float s_mx[kPfRows], s_inv[kPfRows];
+  constexpr int NK = HD / 4, NW = kPfThreads / 64;
+  extern __shared__ __align__(16) float sm[];  // e[16][ld] | cj[16][kPfSegLd] (EXACT)
+  const int ld = pf_ld(t);
+  float *e = sm, *cj = sm + kPfRows * ld;
+  __shared__ __align__(16) float qs[kPfRows * (HD + 4)];
+  __shared__ float s_inv[kPfRows];
   // the exp table in LDS: a per-lane lookup in it does not wait on memory
   __shared__ uint64_t etab[32];
   if (threadIdx.x < 32) etab[threadIdx.x] = syn_exp2_tab[threadIdx.x];
-  const int head = blockIdx.x, i0 = blockIdx.y * kPfRows;
-  const int kvh = head / (nh / nkv);
-  const int qd = nh * hd;
-  const int nrow = min(kPfRows, t - i0);
-  const int tid = threadIdx.x;
-  for (int x = tid; x < kPfRows * hd; x += blockDim.x) {
-    const int r = x / hd, d = x - r * hd;
-    qs[x] = r < nrow ? q[(size_t)(i0 + r) * qd + head * hd + d] : 0.0f;
-  }
-  const float scale = 1.0f / sqrtf((float)hd);
-  // ---- scores: 16 rows x 64 positions per chunk, 4 (row, position) pairs a thread
-  for (int p0 = 0; p0 < t; p0 += kPfChunk) {
-    const int np = min(kPfChunk, t - p0);
-    __syncthreads();  // qs written / the previous chunk consumed
-    // K rows: four consecutive columns are contiguous in the cache layout;
-    // eight 16-byte loads in flight per thread before the LDS stores
-    const int hd4 = hd / 4, nk = np * hd4;
-    for (int x0 = tid; x0 < nk; x0 += 8 * (int)blockDim.x) {
-      float4 v[8];
+  // the last rows see the most positions: start with them
+  const int head = blockIdx.x, i0 = ((int)gridDim.y - 1 - (int)blockIdx.y) * kPfRows;
+  const int kvh = head / (nh / nkv), qd = nh * HD;
+  const int nrow = min(kPfRows, t - i0), nsc = i0 + nrow;  // row r sees i0 + r + 1 <= nsc
+  const int npos = EXACT ? t : nsc;                        // positions of P V
+  const int sh = cache_off & 3;                            // e[r][sh + j]: position j
+  const int tid = threadIdx.x, wave = tid >> 6, m = tid & 15, g = (tid >> 4) & 3;
+  const float scale = 1.0f / sqrtf((float)HD);
+  const float ninf = -__builtin_inff();
+  const int W = (sh + npos + 3) & ~3, steps = W / 4;
+  // V of the first U steps of the wave's first columns: read before the scores,
+  // which hide its latency
+  constexpr int U = 16;
+  const float *vp =
+      vc + kv_v_index(cache_off & ~3, kvh, (wave % (HD / 16)) * 16 + m, HD, max_seq);
+  f32x4 vb[U / 4];
+  auto load_v = [&](int s0) {
 #pragma unroll
-      for (int u = 0; u < 8; u++) {
-        const int x = min(x0 + u * (int)blockDim.x, nk - 1);
-        const int pp = x / hd4, d4 = x - pp * hd4;
-        v[u] = *reinterpret_cast<const float4 *>(
-            kc + kv_k_index(cache_off + p0 + pp, kvh, 4 * d4, hd, max_seq));
-      }
+    for (int u = 0; u < U / 4; u++)
+      vb[u] = *reinterpret_cast<const f32x4 *>(vp + (size_t)min(s0 + 4 * u + g, steps - 1) *
+                                                        (4 * HD));
+  };
+  // ---- scores
+  {
+    const int nt = (nsc + 15) / 16;
+    float qa[NK];
+    f32x4 kb[NK / 4];
+    auto load_k = [&](int tile) {
+      const int p = min(tile * 16 + m, t - 1);
+      const float *kp = kc + kv_k_index(cache_off + p, kvh, 4 * g, HD, max_seq);
 #pragma unroll
-      for (int u = 0; u < 8; u++) {
-        const int x = x0 + u * (int)blockDim.x;
-        if (x < nk) {
-          const int pp = x / hd4, d4 = x - pp * hd4;
-          float *dst = kv + pp * ldk + 4 * d4;
-          dst[0] = v[u].x;
-          dst[1] = v[u].y;
-          dst[2] = v[u].z;
-          dst[3] = v[u].w;
-        }
-      }
-    }
+      for (int i = 0; i < NK / 4; i++) kb[i] = *reinterpret_cast<const f32x4 *>(kp + i * 1024);
+    };
+    // q by way of LDS: read as fragments from memory, 16 rows of 16 bytes a
+    // load, it took longer than all of K
+    f32x4 qv = {0.0f, 0.0f, 0.0f, 0.0f};
+    const int qr = tid / NK, qc = tid % NK * 4;
+    if (qr < kPfRows)
+      qv = *reinterpret_cast<const f32x4 *>(q + (size_t)(i0 + min(qr, nrow - 1)) * qd +
+                                            head * HD + qc);
+    if (wave < nt) load_k(wave);
+    if (wave < HD / 16) load_v(0);
+    __builtin_amdgcn_sched_barrier(0);
+    if (qr < kPfRows) *reinterpret_cast<f32x4 *>(qs + qr * (HD + 4) + qc) = qv;
     __syncthreads();
-    // thread: position pp of the chunk for rows rb, rb+4, rb+8, rb+12 (one K
-    // row read per step, four independent chains; the fused / plain choice
-    // of each chain is a select, so all four keep their own order)
-    const int pp = tid % kPfChunk, rb = tid / kPfChunk;
-    if (pp < np) {
-      const int j = p0 + pp;
-      float acc[4];
-      bool fz[4];
 #pragma unroll
-      for (int u = 0; u < 4; u++) {
-        const int i = i0 + rb + 4 * u;
-        const int tq = (i / 32) * 32, tqs = min(32, t - tq), il = i - tq;
-        fz[u] = sgemm_fused(tqs, il, t, j, true);
-        acc[u] = 0.0f;
-      }
-      const float *kr = kv + pp * ldk;
-      // the four chains usually agree on fused / plain: then one loop form
-      const bool all_f = fz[0] && fz[1] && fz[2] && fz[3];
-      const bool none_f = !fz[0] && !fz[1] && !fz[2] && !fz[3];
-      if (all_f) {
-#pragma unroll 8
-        for (int d = 0; d < hd; d++) {
-          const float kd = kr[d];
+    for (int i = 0; i < NK; i++) qa[i] = qs[m * (HD + 4) + 4 * i + g];
+    for (int tile = wave; tile < nt; tile += NW) {
+      f32x4 kn[NK / 4];
 #pragma unroll
-          for (int u = 0; u < 4; u++) acc[u] = __builtin_fmaf(qs[(rb + 4 * u) * hd + d], kd, acc[u]);
-        }
-      } else if (none_f) {
-#pragma unroll 8
-        for (int d = 0; d < hd; d++) {
-          const float kd = kr[d];
+      for (int i = 0; i < NK / 4; i++) kn[i] = groups_transposed(kb[i]);
+      if (tile + NW < nt) load_k(tile + NW);
+      f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-          for (int u = 0; u < 4; u++) {
-            const float pr = qs[(rb + 4 * u) * hd + d] * kd;
-            acc[u] = acc[u] + pr;
-          }
-        }
-      } else {
-#pragma unroll 8
-        for (int d = 0; d < hd; d++) {
-          const float kd = kr[d];
+      for (int i = 0; i < NK; i++)
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[i], kn[i / 4][i % 4], acc, 0, 0, 0);
+      const int j = tile * 16 + m;
 #pragma unroll
-          for (int u = 0; u < 4; u++) {
-            const float qv = qs[(rb + 4 * u) * hd + d];
-            const float f = __builtin_fmaf(qv, kd, acc[u]);
-            const float pr = qv * kd;
-            const float g = acc[u] + pr;
-            acc[u] = fz[u] ? f : g;
-          }
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < 4; u++) {
-        const int r = rb + 4 * u, i = i0 + r;
-        if (r < nrow) {
-          float sc = acc[u] * scale;
-          if (j > i) sc = -__builtin_inff();
-          e[r * t + j] = sc;
-        }
+      for (int r = 0; r < 4; r++) {
+        const int row = 4 * g + r;
+        if (j < nsc) e[row * ld + sh + j] = j <= i0 + row ? acc[r] * scale : ninf;
       }
     }
   }
   __syncthreads();
-  // ---- online max / sum per row (k_attn_prefill's order): 16 threads a row
-  // precompute the exponentials over contiguous chunks, one thread a row
-  // runs the dependent chain
-  {
-    const int r = tid / 16, part = tid % 16;
-    const int per = (t + 15) / 16;
-    const int j0 = min(part * per, t), j1 = min(j0 + per, t);
-    float *er = e + r * t, *cr = cj + r * t;
-    float lm = -__builtin_inff();
-    if (r < nrow)
-      for (int j = j0; j < j1; j++) lm = fmaxf(lm, er[j]);
-    // exclusive prefix of the chunk maxima within the 16-lane group
-    float run = -__builtin_inff(), all = -__builtin_inff();
-    for (int o = 0; o < 16; o++) {
-      const float v = __shfl(lm, (tid & ~15) + o);
-      if (o < part) run = fmaxf(run, v);
-      all = fmaxf(all, v);
-    }
-    if (r < nrow)
-      for (int j = j0; j < j1; j++) {
-        const float x = er[j];
-        cr[j] = x > run ? -syn_expf_tab(run - x, etab) : syn_expf_tab(x - run, etab);
-        run = fmaxf(run, x);
-      }
-    __syncthreads();
-    if (part == 0 && r < nrow) {
-      float se = 0.0f;
-      int j = 0;
-      for (; j + 8 <= t; j += 8) {
-        float c[8];
+  // rows from r_plain on are the reference's partial micro-tile (plain a*b + c)
+  const int tq = i0 & ~31, tqs = min(32, t - tq);
+  const int r_plain =
+      EXACT && tqs > 16 ? min(nrow, max(0, (tqs & ~7) - (i0 - tq))) : nrow;
+  if constexpr (EXACT) {
+    auto plain = [&](int r, int j) {
+      const float *qr = q + (size_t)(i0 + r) * qd + head * HD;
+      const float *kp = kc + kv_k_index(cache_off + j, kvh, 0, HD, max_seq);
+      float acc = 0.0f;
+#pragma unroll 8
+      for (int d4 = 0; d4 < NK; d4++) {
+        const f32x4 a = *reinterpret_cast<const f32x4 *>(qr + 4 * d4);
+        const f32x4 b = *reinterpret_cast<const f32x4 *>(kp + d4 * 256);
 #pragma unroll
-        for (int u = 0; u < 8; u++) c[u] = cr[j + u];
+        for (int u = 0; u < 4; u++) {
+          const float p = a[u] * b[u];
+          acc = acc + p;
+        }
+      }
+      e[r * ld + sh + j] = acc * scale;
+    };
+    for (int x = tid; x < (nrow - r_plain) * nsc; x += kPfThreads) {
+      const int r = r_plain + x / nsc, j = x % nsc;
+      if (j <= i0 + r) plain(r, j);
+    }
+    const int tc = t & 7;  // the last t % 8 columns
+    if (nsc > t - tc)
+      for (int x = tid; x < r_plain * tc; x += kPfThreads) {
+        const int r = x / tc, j = t - tc + x % tc;
+        if (j <= i0 + r) plain(r, j);
+      }
+    if (r_plain < nrow || nsc > t - tc) __syncthreads();
+  }
+  // ---- softmax: 32 threads a row
+  {
+    const int r = tid >> 5, part = tid & 31;
+    const int vis = r < nrow ? i0 + r + 1 : 0;
+    float *er = e + r * ld + sh;
+    float mx = ninf, inv = 0.0f;
+    if constexpr (EXACT) {
+      // k_attn_prefill's order: at position j the running maximum is that of
+      // the positions before it, so every exponential is known up front
+      float se = 0.0f, *cr = cj + r * kPfSegLd;
+      for (int s0 = 0; s0 < nsc; s0 += kPfSeg) {
+        const int per = (min(kPfSeg, nsc - s0) + 31) / 32;
+        const int j0 = min(s0 + part * per, vis), j1 = min(j0 + per, vis);
+        float x[8], lm = ninf;
 #pragma unroll
         for (int u = 0; u < 8; u++) {
-          const float cu = fabsf(c[u]);
-          const float pr = se * cu;
-          se = __builtin_signbit(c[u]) ? pr + 1.0f : se + cu;
+          x[u] = u < per && j0 + u < j1 ? er[j0 + u] : ninf;
+          lm = fmaxf(lm, x[u]);
         }
-      }
-      for (; j < t; j++) {
-        const float cu = fabsf(cr[j]);
-        const float pr = se * cu;
-        se = __builtin_signbit(cr[j]) ? pr + 1.0f : se + cu;
-      }
-      s_mx[r] = all;
-      s_inv[r] = 1.0f / se;
-    }
-    __syncthreads();
-  }
-  for (int x = tid; x < nrow * t; x += blockDim.x) {
-    const int r = x / t;
-    e[x] = syn_expf_tab(e[x] - s_mx[r], etab) * s_inv[r];
-  }
-  // ---- P V: 16 rows x hd columns, chains over the positions in order.
-  // hd divides 256: thread = column d for rows r0, r0 + 256/hd, ... (one V
-  // read per position, hd/16 independent chains)
-  const int d = tid % hd, rstep = (int)blockDim.x / hd, r0 = tid / hd, nch = kPfRows / rstep;
-  constexpr int kMaxPer = 8;
-  float acc[kMaxPer];
-  bool fz[kMaxPer];
-#pragma unroll
-  for (int u = 0; u < kMaxPer; u++) {
-    const int i = i0 + r0 + u * rstep;
-    const int tq = (i / 32) * 32, tqs = min(32, t - tq), il = i - tq;
-    fz[u] = sgemm_fused(tqs, il, hd, d, false);
-    acc[u] = 0.0f;
-  }
-  for (int p0 = 0; p0 < t; p0 += kPfChunk) {
-    const int np = min(kPfChunk, t - p0);
-    __syncthreads();
-    const int nv = np * hd;  // eight loads in flight per thread
-    for (int x0 = tid; x0 < nv; x0 += 8 * (int)blockDim.x) {
-      float v[8];
-#pragma unroll
-      for (int u = 0; u < 8; u++) {
-        const int x = min(x0 + u * (int)blockDim.x, nv - 1);
-        const int pp = x / hd, dd = x - pp * hd;
-        v[u] = vc[kv_v_index(cache_off + p0 + pp, kvh, dd, hd, max_seq)];
-      }
-#pragma unroll
-      for (int u = 0; u < 8; u++) {
-        const int x = x0 + u * (int)blockDim.x;
-        if (x < nv) {
-          const int pp = x / hd, dd = x - pp * hd;
-          kv[pp * ldk + dd] = v[u];
+        for (int o = 1; o < 32; o <<= 1) {  // maxima of the parts up to this one
+          const float v = __shfl_up(lm, o, 32);
+          if (part >= o) lm = fmaxf(lm, v);
         }
-      }
-    }
-    __syncthreads();
-    bool all_f = true, none_f = true;
+        float run = __shfl_up(lm, 1, 32);
+        run = part == 0 ? mx : fmaxf(mx, run);
+        mx = fmaxf(mx, __shfl(lm, 31, 32));
 #pragma unroll
-    for (int u = 0; u < kMaxPer; u++)
-      if (u < nch) {
-        all_f = all_f && fz[u];
-        none_f = none_f && !fz[u];
-      }
-    if (all_f) {
-#pragma unroll 4
-      for (int pp = 0; pp < np; pp++) {
-        const float v = kv[pp * ldk + d];
+        for (int u0 = 0; u0 < 8; u0 += 4)
+          if (u0 < per) {
+            float c[4];
 #pragma unroll
-        for (int u = 0; u < kMaxPer; u++)
-          if (u < nch) acc[u] = __builtin_fmaf(e[(r0 + u * rstep) * t + p0 + pp], v, acc[u]);
-      }
-    } else if (none_f) {
-#pragma unroll 4
-      for (int pp = 0; pp < np; pp++) {
-        const float v = kv[pp * ldk + d];
+            for (int u = 0; u < 4; u++) {
+              const float y = x[u0 + u];
+              const bool up = y > run;
+              const float ex = syn_expf_sel(up ? run - y : y - run, etab);
+              // (past the row's positions: 0, without effect on the chain)
+              c[u] = j0 + u0 + u < j1 ? (up ? -ex : ex) : 0.0f;
+              run = fmaxf(run, y);
+            }
 #pragma unroll
-        for (int u = 0; u < kMaxPer; u++)
-          if (u < nch) {
-            const float m = e[(r0 + u * rstep) * t + p0 + pp] * v;
-            acc[u] = acc[u] + m;
+            for (int u = 0; u < 4; u++)
+              if (u0 + u < per) cr[part * per + u0 + u] = c[u];
           }
+        __syncthreads();
+        if (part == 0) {
+          const int n = min(kPfSeg, vis - s0);
+          auto link = [&](float c) {
+            const float cu = fabsf(c), pr = se * cu;
+            se = __builtin_signbit(c) ? pr + 1.0f : se + cu;
+          };
+          f32x4 na = *reinterpret_cast<const f32x4 *>(cr);
+          f32x4 nb = *reinterpret_cast<const f32x4 *>(cr + 4);
+          for (int j = 0; j < n; j += 8) {
+            const f32x4 a = na, b = nb;  // (the next eight: at most the row's padding)
+            na = *reinterpret_cast<const f32x4 *>(cr + min(j + 8, kPfSegLd - 8));
+            nb = *reinterpret_cast<const f32x4 *>(cr + min(j + 12, kPfSegLd - 4));
+            const bool neg = __builtin_signbit(a.x) | __builtin_signbit(a.y) |
+                             __builtin_signbit(a.z) | __builtin_signbit(a.w) |
+                             __builtin_signbit(b.x) | __builtin_signbit(b.y) |
+                             __builtin_signbit(b.z) | __builtin_signbit(b.w);
+            if (neg) {
+#pragma unroll
+              for (int u = 0; u < 4; u++) link(a[u]);
+#pragma unroll
+              for (int u = 0; u < 4; u++) link(b[u]);
+            } else {  // no new maximum: additions only
+#pragma unroll
+              for (int u = 0; u < 4; u++) se = se + a[u];
+#pragma unroll
+              for (int u = 0; u < 4; u++) se = se + b[u];
+            }
+          }
+        }
+        __syncthreads();
       }
+      inv = 1.0f / __shfl(se, 0, 32);
+      // (masked positions: 0 * inv)
+      for (int j0 = part; j0 < vis; j0 += 128) {
+        float v[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+          v[u] = syn_expf_sel(er[min(j0 + 32 * u, vis - 1)] - mx, etab) * inv;
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+          if (j0 + 32 * u < vis) er[j0 + 32 * u] = v[u];
+      }
+      if (part < sh) er[part - sh] = 0.0f;
+      for (int j = vis + part; j < W - sh; j += 32)
+        er[j] = r < nrow && j < npos ? 0.0f * inv : 0.0f;
     } else {
-#pragma unroll 4
-      for (int pp = 0; pp < np; pp++) {
-        const float v = kv[pp * ldk + d];
+      for (int j = part; j < vis; j += 32) mx = fmaxf(mx, er[j]);
+      for (int o = 1; o < 32; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+      float sum = 0.0f;
+      for (int j0 = part; j0 < vis; j0 += 128) {
+        float v[4];
 #pragma unroll
-        for (int u = 0; u < kMaxPer; u++) {
-          if (u < nch) {
-            const float ev = e[(r0 + u * rstep) * t + p0 + pp];
-            const float f = __builtin_fmaf(ev, v, acc[u]);
-            const float m = ev * v;
-            const float g = acc[u] + m;
-            acc[u] = fz[u] ? f : g;
+        for (int u = 0; u < 4; u++) v[u] = syn_expf_sel(er[min(j0 + 32 * u, vis - 1)] - mx, etab);
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+          if (j0 + 32 * u < vis) {
+            er[j0 + 32 * u] = v[u];
+            sum += v[u];
           }
-        }
       }
-    }
-  }
-#pragma unroll
-  for (int u = 0; u < kMaxPer; u++) {
-    const int r = r0 + u * rstep;
-    if (u < nch && r < nrow) out[(size_t)(i0 + r) * qd + head * hd + d] = acc[u];
-  }
-}
-
-// Prefill attention for the tolerance-graded decoders (K-quant): the same
-// causal attention over the prompt block (row i sees positions 0 .. i of
-// the t new ones at cache_off), without the reference's serial order.  One
-// workgroup per (head, 32 query rows); K, then V, staged through LDS 64
-// positions at a time in rows padded to HD + 4 floats (16-byte aligned,
-// rows four banks apart).  Eight threads per query row: thread c8 of row r
-// takes positions c8 + 8k of a chunk (eight independent FMA chains over
-// d), the row's max and sum by shuffles over its 8 lanes, then the output
-// columns c8 + 8k (HD / 8 chains over the positions; contiguous columns per
-// thread with 16-byte reads of V measured slower, 86.6 against 76.4 us at
-// LLaMA-3B, 256 tokens).  The scores of the
-// block's rows stay in LDS (32 x t floats).
-constexpr int kPtRows = 32, kPtChunk = 64;
-
-template <int HD>
-__global__ void __launch_bounds__(256)
-    k_attn_prefill_tile(const float *__restrict__ q, const float *__restrict__ kc,
-                        const float *__restrict__ vc, int t, int nh, int nkv, int max_seq,
-                        int cache_off, float *__restrict__ out) {
-  constexpr int LD = HD + 4, HD4 = HD / 4, NCOL = HD / 8;
-  constexpr int KL = kPtChunk * HD4 / 256, VL = (17 * HD + 255) / 256;  // loads per thread
-  extern __shared__ __align__(16) float smt[];
-  const int tps = ((t + 3) & ~3) + 1;  // odd score-row stride
-  float *qs = smt, *kv = qs + kPtRows * LD, *S = kv + kPtChunk * LD;
-  __shared__ float s_inv[kPtRows];
-  const int head = blockIdx.x, i0 = blockIdx.y * kPtRows;
-  const int kvh = head / (nh / nkv), qd = nh * HD;
-  const int nrow = min(kPtRows, t - i0), npos = i0 + nrow;
-  const int tid = threadIdx.x, r = tid >> 3, c8 = tid & 7;
-  for (int x = tid; x < kPtRows * HD; x += 256) {
-    const int rr = x / HD, d = x - rr * HD;
-    qs[rr * LD + d] = rr < nrow ? q[(size_t)(i0 + rr) * qd + head * HD + d] : 0.0f;
-  }
-  const float scale = 1.0f / sqrtf((float)HD);
-  const f32x4 *q4 = reinterpret_cast<const f32x4 *>(qs + r * LD);
-  // ---- scores
-  for (int p0 = 0; p0 < npos; p0 += kPtChunk) {
-    const int np = min(kPtChunk, npos - p0);
-    // K rows: 16 bytes (four consecutive d) per load, all issued before
-    // the barrier and the LDS stores; positions past np are stored as zeros
-    f32x4 kr[KL];
-#pragma unroll
-    for (int i = 0; i < KL; i++) {
-      const int x = tid + 256 * i, p = min(x & 63, np - 1), d4 = x >> 6;
-      kr[i] = *reinterpret_cast<const f32x4 *>(
-          kc + kv_k_index(cache_off + p0 + p, kvh, d4 * 4, HD, max_seq));
-    }
-    __syncthreads();  // qs written / the previous chunk consumed
-#pragma unroll
-    for (int i = 0; i < KL; i++) {
-      const int x = tid + 256 * i, p = x & 63, d4 = x >> 6;
-      *reinterpret_cast<f32x4 *>(kv + p * LD + d4 * 4) = p < np ? kr[i] : f32x4{0, 0, 0, 0};
-    }
-    __syncthreads();
-    float acc[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll 4
-    for (int d4 = 0; d4 < HD4; d4++) {
-      const f32x4 a = q4[d4];
-#pragma unroll
-      for (int k = 0; k < 8; k++) {
-        const f32x4 b = reinterpret_cast<const f32x4 *>(kv + (c8 + 8 * k) * LD)[d4];
-        acc[k] = __builtin_fmaf(a.x, b.x, acc[k]);
-        acc[k] = __builtin_fmaf(a.y, b.y, acc[k]);
-        acc[k] = __builtin_fmaf(a.z, b.z, acc[k]);
-        acc[k] = __builtin_fmaf(a.w, b.w, acc[k]);
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < 8; k++) {
-      const int p = p0 + c8 + 8 * k;
-      if (p < npos) S[r * tps + p] = p <= i0 + r ? acc[k] * scale : -__builtin_inff();
+      if (part < sh) er[part - sh] = 0.0f;
+      for (int j = vis + part; j < W - sh; j += 32) er[j] = 0.0f;
+      for (int o = 1; o < 32; o <<= 1) sum += __shfl_xor(sum, o);
+      if (part == 0) s_inv[r] = 1.0f / sum;
     }
   }
   __syncthreads();
-  // ---- softmax of row r (positions 0 .. npos-1; masked ones are -inf)
-  float mx = -__builtin_inff();
-  for (int p = c8; p < npos; p += 8) mx = fmaxf(mx, S[r * tps + p]);
-  mx = fmaxf(mx, __shfl_xor(mx, 1));
-  mx = fmaxf(mx, __shfl_xor(mx, 2));
-  mx = fmaxf(mx, __shfl_xor(mx, 4));
-  float sum = 0.0f;
-  for (int p = c8; p < npos; p += 8) {
-    const float e = syn_expf(S[r * tps + p] - mx);
-    S[r * tps + p] = e;
-    sum += e;
-  }
-  sum += __shfl_xor(sum, 1);
-  sum += __shfl_xor(sum, 2);
-  sum += __shfl_xor(sum, 4);
-  if (c8 == 0) s_inv[r] = 1.0f / sum;
-  // ---- P.V
-  float o[NCOL];
+  // ---- P V
+  const int r_plain_v = EXACT && HD == 16 && tqs <= 16 ? 0 : r_plain;
+  static_assert(HD / 16 <= NW, "one group of columns a wave");
+  if (wave < HD / 16) {
+    const int ct = wave;
+    const float *ep = e + m * ld + g;
+    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int s0 = 0; s0 < steps; s0 += U) {
+      f32x4 vn[U / 4];
 #pragma unroll
-  for (int k = 0; k < NCOL; k++) o[k] = 0.0f;
-  for (int p0 = 0; p0 < npos; p0 += kPtChunk) {
-    const int np = min(kPtChunk, npos - p0);
-    // V: 16 bytes (four consecutive positions of one d) per load, from the
-    // aligned group holding position cache_off + p0 on: ng <= 17 groups
-    const int P0 = cache_off + p0, g0 = P0 >> 2, ng = ((P0 + np - 1) >> 2) - g0 + 1;
-    f32x4 vr[VL];
+      for (int u = 0; u < U / 4; u++) {
+        const int j = 4 * (s0 + 4 * u + g) - sh;
+        f32x4 v = vb[u];
 #pragma unroll
-    for (int i = 0; i < VL; i++) {
-      const int x = tid + 256 * i, gi = min(x / HD, ng - 1), d = x % HD;
-      vr[i] = *reinterpret_cast<const f32x4 *>(vc + kv_v_index(4 * (g0 + gi), kvh, d, HD, max_seq));
-    }
-    __syncthreads();  // scores and s_inv written / the previous chunk consumed
-#pragma unroll
-    for (int i = 0; i < VL; i++) {
-      const int x = tid + 256 * i, gi = x / HD, d = x % HD;
-      if (gi < ng) {
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-          const int lp = 4 * (g0 + gi) + j - P0;
-          if (lp >= 0 && lp < np) kv[lp * LD + d] = vr[i][j];
-        }
+        for (int c = 0; c < 4; c++) v[c] = j + c >= 0 && j + c < npos ? v[c] : -0.0f;
+        vn[u] = groups_transposed(v);
       }
-    }
-    __syncthreads();
-    const float *srow = S + r * tps + p0;
-    for (int p = 0; p < np; p++) {
-      const float e = srow[p];
-      const float *vr = kv + p * LD + c8;
+      if (s0 + U < steps) load_v(s0 + U);
+      float a[U];
 #pragma unroll
-      for (int k = 0; k < NCOL; k++) o[k] = __builtin_fmaf(e, vr[8 * k], o[k]);
+      for (int u = 0; u < U; u++) a[u] = ep[4 * min(s0 + u, steps - 1)];
+#pragma unroll
+      for (int u = 0; u < U; u++)
+        if (s0 + u < steps)
+          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u], vn[u / 4][u % 4], acc, 0, 0, 0);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int row = 4 * g + r;
+      if (row < r_plain_v || (!EXACT && row < nrow))
+        out[(size_t)(i0 + row) * qd + head * HD + ct * 16 + m] =
+            EXACT ? acc[r] : acc[r] * s_inv[row];
     }
   }
-  if (r < nrow) {
-    const float inv = s_inv[r];
-#pragma unroll
-    for (int k = 0; k < NCOL; k++) out[(size_t)(i0 + r) * qd + head * HD + c8 + 8 * k] = o[k] * inv;
+  if constexpr (EXACT) {
+    for (int x = tid; x < (nrow - r_plain_v) * HD; x += kPfThreads) {
+      const int r = r_plain_v + x / HD, d = x % HD;
+      const float *er = e + r * ld + sh;
+      float acc = 0.0f;
+#pragma unroll 8
+      for (int j = 0; j < t; j++) {
+        const float p = er[j] * vc[kv_v_index(cache_off + j, kvh, d, HD, max_seq)];
+        acc = acc + p;
+      }
+      out[(size_t)(i0 + r) * qd + head * HD + d] = acc;
+    }
   }
 }
 
-static size_t attn_prefill_tile_lds(int hd, int t) {
-  return ((size_t)(kPtRows + kPtChunk) * (hd + 4) + (size_t)kPtRows * (((t + 3) & ~3) + 1)) *
-         sizeof(float);
-}
-
-syn_status_t launch_attention_prefill_tol(const float *q, const float *kcache,
-                                          const float *vcache, int t, int n_heads, int n_kv,
-                                          int head_dim, int max_seq, float *out, hipStream_t s,
-                                          int cache_off) {
-  const size_t shm = attn_prefill_tile_lds(head_dim, t);
-  if (!(head_dim == 16 || head_dim == 32 || head_dim == 64 || head_dim == 128) ||
-      shm > 144 * 1024)
-    return launch_attention_prefill(q, kcache, vcache, t, n_heads, n_kv, head_dim, max_seq,
-                                    nullptr, out, s, cache_off);
+// the matrix-core kernel for head widths of 16, 32, 64 and 128 whose rows of
+// scores fit LDS; *done says whether it took the call
+template <bool EXACT>
+static syn_status_t launch_prefill_mfma(const float *q, const float *kcache, const float *vcache,
+                                        int t, int n_heads, int n_kv, int head_dim, int max_seq,
+                                        int cache_off, float *out, hipStream_t s, bool *done) {
+  const size_t shm =
+      ((size_t)kPfRows * pf_ld(t) + (EXACT ? kPfRows * kPfSegLd : 0)) * sizeof(float);
+  *done = (head_dim == 16 || head_dim == 32 || head_dim == 64 || head_dim == 128) &&
+          shm <= 144 * 1024;
+  if (!*done) return SYN_OK;
   static bool attr[4] = {false, false, false, false};
   auto run = [&](auto kern, int which) -> syn_status_t {
     if (!attr[which]) {  // more than the default 64 KiB of dynamic LDS
@@ -846,47 +770,42 @@ syn_status_t launch_attention_prefill_tol(const float *q, const float *kcache,
                                   144 * 1024));
       attr[which] = true;
     }
-    SYN_LAUNCH(kern, dim3(n_heads, (t + kPtRows - 1) / kPtRows), dim3(256), shm, s, q, kcache,
-               vcache, t, n_heads, n_kv, max_seq, cache_off, out);
+    SYN_LAUNCH(kern, dim3(n_heads, (t + kPfRows - 1) / kPfRows), dim3(kPfThreads), shm, s, q,
+               kcache, vcache, t, n_heads, n_kv, max_seq, cache_off, out);
     SYN_LAUNCH_CHECK();
     return SYN_OK;
   };
   switch (head_dim) {
-    case 16: return run(k_attn_prefill_tile<16>, 0);
-    case 32: return run(k_attn_prefill_tile<32>, 1);
-    case 64: return run(k_attn_prefill_tile<64>, 2);
-    default: return run(k_attn_prefill_tile<128>, 3);
+    case 16: return run(k_attn_prefill_mfma<16, EXACT>, 0);
+    case 32: return run(k_attn_prefill_mfma<32, EXACT>, 1);
+    case 64: return run(k_attn_prefill_mfma<64, EXACT>, 2);
+    default: return run(k_attn_prefill_mfma<128, EXACT>, 3);
   }
+}
+
+// For the tolerance-graded decoders (K-quant, hybrid): the same causal
+// attention over the prompt block (row i sees positions 0 .. i of the t new
+// ones at cache_off), without the reference's serial order of the sum.
+syn_status_t launch_attention_prefill_tol(const float *q, const float *kcache,
+                                          const float *vcache, int t, int n_heads, int n_kv,
+                                          int head_dim, int max_seq, float *out, hipStream_t s,
+                                          int cache_off) {
+  bool done;
+  SYN_TRY(launch_prefill_mfma<false>(q, kcache, vcache, t, n_heads, n_kv, head_dim, max_seq,
+                                     cache_off, out, s, &done));
+  if (done) return SYN_OK;
+  return launch_attention_prefill(q, kcache, vcache, t, n_heads, n_kv, head_dim, max_seq, nullptr,
+                                  out, s, cache_off);
 }
 
 syn_status_t launch_attention_prefill(const float *q, const float *kcache, const float *vcache,
                                       int t, int n_heads, int n_kv, int head_dim, int max_seq,
                                       float *scores, float *out, hipStream_t s, int cache_off) {
   (void)scores;
-  // row-block kernel when its LDS rows fit (hd <= 128: 8 outputs a thread)
-  const size_t shm_rows = (size_t)(kPfRows * head_dim + kPfChunk * (head_dim + 1) +
-                                   2 * kPfRows * t) * sizeof(float);
-  if ((head_dim == 16 || head_dim == 32 || head_dim == 64 || head_dim == 128) &&
-      shm_rows <= 144 * 1024) {
-    static bool attr_rows[4] = {false, false, false, false};
-    auto run = [&](auto kern, int which) -> syn_status_t {
-      if (!attr_rows[which]) {
-        SYN_HIP(hipFuncSetAttribute((const void *)kern,
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, 144 * 1024));
-        attr_rows[which] = true;
-      }
-      hipLaunchKernelGGL(kern, dim3(n_heads, (t + kPfRows - 1) / kPfRows), dim3(256), shm_rows,
-                         s, q, kcache, vcache, t, n_heads, n_kv, max_seq, cache_off, out);
-      SYN_LAUNCH_CHECK();
-      return SYN_OK;
-    };
-    switch (head_dim) {
-      case 16: return run(k_attn_prefill_rows<16>, 0);
-      case 32: return run(k_attn_prefill_rows<32>, 1);
-      case 64: return run(k_attn_prefill_rows<64>, 2);
-      default: return run(k_attn_prefill_rows<128>, 3);
-    }
-  }
+  bool done;
+  SYN_TRY(launch_prefill_mfma<true>(q, kcache, vcache, t, n_heads, n_kv, head_dim, max_seq,
+                                    cache_off, out, s, &done));
+  if (done) return SYN_OK;
   const size_t shm = (size_t)(head_dim + 2 * t) * sizeof(float);
   if (shm > 144 * 1024) {
     set_error("prefill attention: prompt too long for one workgroup's LDS rows");

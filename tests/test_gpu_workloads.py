@@ -7,7 +7,7 @@ the head_dim-128 prefill attention bit for bit.
 - Config 3 (LLaMA-3.2-3B widths, Q4_K attention and gate/up, Q6_K down and
   lm_head): four layers at full width with the 256-token prompt and 128
   decode steps against the oracle's f32 CausalLM (cosine >= 0.9999 at every
-  step: the prefill runs the f16 MFMA GEMM and k_attn_prefill_rows<128> on
+  step: the prefill runs the f16 MFMA GEMM and k_attn_prefill_mfma<128> on
   256 rows, the decode attention runs at positions 256-383); and the full
   28-layer model through properties (finite logits; the prefill of n tokens
   matches the prefill of n - 1 followed by forward_one).
