@@ -66,7 +66,7 @@ _STEP_KIB = {"qkv": (2157.1, 68.0), "attention": (377.5, 32.0), "o": (1078.0, 64
              "gate_up": (3206.6, 113.5), "down": (1605.5, 48.0)}
 STEP_SOURCES = ("synapse_amd/csrc/decode_fused.hip", "synapse_amd/csrc/fused_dev.hpp",
                 "synapse_amd/csrc/qlm.hip")
-STEP_SOURCES_SHA16 = "43f9074b6c63b25e"
+STEP_SOURCES_SHA16 = "063e45eee3fd6013"
 
 
 def step_sources_sha16() -> str:
