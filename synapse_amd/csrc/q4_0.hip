@@ -343,7 +343,7 @@ syn_status_t QLinearQ4_0::gemv(size_t m, const float *d_x, size_t ldx, float *d_
   // -> 2048 13-15 against 9).  7 and 8 rows only on large matrices (8 rows,
   // 3072 -> 8192 18.6 against 12, 14336 -> 4096 38 against 30; 4096 -> 1024
   // 9.0 against 12.5)
-  if (gemm_ok() && ldx % 4 == 0 && m <= 16 && (m >= 9 || (m >= 7 && n * k >= 24000000)))
+  if (split_ok() && ldx % 4 == 0 && m <= 16 && (m >= 9 || (m >= 7 && n * k >= 24000000)))
     return gemm_split(m, d_x, ldx, d_y, ldy, s);
   const float sub = rs_f16_scales ? 0.5f : 1.0f;
   // "chunks" here are 32-element blocks; a K slice holds whole blocks.  One
@@ -432,7 +432,7 @@ syn_status_t QLinearQ4_0::upload_packed(const uint8_t *packed, size_t n_, size_t
   const size_t P = cdiv(n_, 64), B = (size_t)blocks;
   std::vector<uint8_t> hn(P * B * 64 * 16, 0x88);  // padding rows: nibble 8 -> value 0
   std::vector<uint16_t> hs(P * B * 64, 0);
-  has_subnormal_scale = false;
+  has_subnormal_scale = has_wide_scale = false;
   for (size_t row = 0; row < n_; row++) {
     const size_t p = row / 64, r = row % 64;
     for (size_t b = 0; b < B; b++) {
@@ -440,6 +440,7 @@ syn_status_t QLinearQ4_0::upload_packed(const uint8_t *packed, size_t n_, size_t
       const uint16_t d = (uint16_t)(src[0] | (src[1] << 8));
       hs[(p * B + b) * 64 + r] = d;
       if ((d & 0x7c00u) == 0 && (d & 0x3ffu) != 0) has_subnormal_scale = true;
+      if ((d & 0x7fffu) > 0x6fffu) has_wide_scale = true;  // |d| >= 2^13
       std::memcpy(&hn[((p * B + b) * 64 + r) * 16], src + 2, 16);
     }
   }

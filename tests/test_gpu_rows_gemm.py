@@ -103,10 +103,31 @@ def test_split_rows_extremes():
     got = lin.forward(x)
     with np.errstate(invalid="ignore"):
         want = x.astype(np.float64) @ w.T
+        inf_row = (np.inf * w[:, 7]).astype(np.float32)
     assert not got[1].any()
-    assert np.isnan(got[5]).all() and not np.isfinite(got[4]).any()
+    assert np.isnan(got[5]).all()
+    # infinity times a weight of zero is a NaN, else an infinity of its sign
+    np.testing.assert_array_equal(got[4], inf_row)
     for r in (0, 2, 3, 6, 7, 8, 9, 10, 11):
         size = np.abs(x[r]).astype(np.float64) @ np.abs(w).T
         # subnormal outputs round to 2^-149
         assert (np.abs(got[r] - want[r]) <= 1e-6 * size + 2.0**-148).all(), r
+    lin.close()
+
+
+@pytest.mark.parametrize("d", [2.0**13, 65504.0])
+def test_wide_scales_keep_the_gemv(d):
+    # 8 d beyond f16: the rows stay on the f32 GEMV
+    n, k, m = 64, 512, 12
+    rng = np.random.default_rng(21)
+    raw = rng.integers(0, 256, (n * k // 32, 18), dtype=np.uint8)
+    dd = np.full(n * k // 32, 0.01, np.float16)
+    dd[5] = d
+    raw[:, :2] = dd.view(np.uint8).reshape(-1, 2)
+    raw[5, 2] = 0x00  # nibble 0: -8 d
+    q = np.empty((n * k // 32, 32))
+    q[:, 0::2], q[:, 1::2] = raw[:, 2:] & 15, raw[:, 2:] >> 4
+    w = ((q - 8) * dd.astype(np.float64)[:, None]).reshape(n, k)
+    lin = hip.QLinear.q4_0(raw.reshape(-1), n, k)
+    _check(lin, w, rng.standard_normal((m, k)).astype(np.float32), True)
     lin.close()
