@@ -391,8 +391,11 @@ syn_status_t QLinearInt8::gemv(size_t m, const int8_t *d_xq, size_t ldx, const f
 // workgroups per CU (each repeats the maximum: 1024 -> 32768, 512 workgroups,
 // 9.2 to 7.2 us; a vocabulary's 2374 would repeat it nine times over).  Two
 // rows double that work: 4096 -> 4096 8.5 us against 8.4 in two launches.
-bool QLinearInt8::forward_fits(size_t m, const float *d_x) const {
+// Every workgroup reads all of x, so y may not overlap it (in two launches it
+// may: the quantizer ends before y is written).
+bool QLinearInt8::forward_fits(size_t m, const float *d_x, const float *d_y) const {
   if (m != 1 || n == 0 || k == 0 || k % 4 || k > 16384 || (uintptr_t)d_x % 16) return false;
+  if (ranges_overlap(d_x, k * sizeof(float), d_y, n * sizeof(float))) return false;
   const GemvPlan p = make_gemv_plan(n, (size_t)chunks, false);
   return p.panels * p.ksplit <= 512;
 }
@@ -651,7 +654,7 @@ syn_status_t syn_hip_qlinear_forward(syn_hip_qlinear_t *h, size_t m, const float
   if (h->fmt == SYN_HIP_FMT_TERNARY) return h->ter.gemv(m, d_x, h->ter.k, d_y, h->ter.n, s);
   if (h->fmt != SYN_HIP_FMT_INT8) return SYN_ERR_INVALID_ARG;
   QLinearInt8 &L = h->i8;
-  if (L.forward_fits(m, d_x)) return L.forward_f32(d_x, d_y, s);
+  if (L.forward_fits(m, d_x, d_y)) return L.forward_f32(d_x, d_y, s);
   const size_t ldq = (size_t)L.chunks * 16;
   if (L.xq_rows < m) {
     SYN_HIP(hipDeviceSynchronize());

@@ -954,8 +954,12 @@ static syn_status_t kq_gemm_f16(int fmt, bool exact, const u32x4 *W, const uint1
     g.blocks = blocks;
     g.n = n;
     g.k = k;
-    // K splits add into rows that the conversion clears 16 bytes at a time
-    const bool can_split = ldy % 4 == 0 && reinterpret_cast<uintptr_t>(d_y) % 16 == 0;
+    // K splits add into rows that the conversion clears 16 bytes at a time,
+    // while it still reads x
+    const bool can_split =
+        ldy % 4 == 0 && reinterpret_cast<uintptr_t>(d_y) % 16 == 0 &&
+        !ranges_overlap(d_x, ((m - 1) * ldx + k) * sizeof(float), d_y,
+                        ((m - 1) * ldy + n) * sizeof(float));
     const int kz = can_split ? rows_gemm_splits(g, m, false) : 1;
     SYN_TRY(ensure_rows(f16_rows_bytes(m, k), xh, xh_bytes));
     SYN_TRY(launch_rows_frag(fmt, d_x, ldx, m, k, false, xh.p, kz > 1 ? d_y : nullptr, ldy, n, s));

@@ -28,6 +28,11 @@ struct GemvPlan {
 
 GemvPlan make_gemv_plan(size_t n, size_t k_chunks, bool chunked_kc);
 
+inline bool ranges_overlap(const void *a, size_t a_bytes, const void *b, size_t b_bytes) {
+  const uintptr_t p = reinterpret_cast<uintptr_t>(a), q = reinterpret_cast<uintptr_t>(b);
+  return p < q + b_bytes && q < p + a_bytes;
+}
+
 // INT8 W8A8 linear: QuantizedLinear (quantization/primitives/int8_linear.rs)
 struct QLinearInt8 {
   size_t n = 0, k = 0;
@@ -62,7 +67,7 @@ struct QLinearInt8 {
                          float *d_y, size_t ldy, int *d_part, hipStream_t s);
   size_t part_elems_for(size_t m) const;
   // y = forward of one f32 row in one launch, quantized inside
-  bool forward_fits(size_t m, const float *d_x) const;
+  bool forward_fits(size_t m, const float *d_x, const float *d_y) const;
   syn_status_t forward_f32(const float *d_x, float *d_y, hipStream_t s);
   syn_status_t ensure_part(size_t elems);
   // allocate split-K scratch for up to max_m activation rows (needed before

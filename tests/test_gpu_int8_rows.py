@@ -80,3 +80,21 @@ def test_one_launch_forward(k, n):
         a2, _ = _both(lin, x)  # the K split's accumulators were left clear
         np.testing.assert_array_equal(a2, b)
     lin.close()
+
+
+def test_forward_in_place():
+    # y over x: every row is quantized before any of y is written
+    n = k = 4096
+    rng = np.random.default_rng(6)
+    lin = hip.QLinear.int8(rng.integers(-128, 128, (n, k), dtype=np.int8),
+                           (rng.random(n) * 1e-3 + 1e-4).astype(np.float32), hip.LAYOUT_NK)
+    x = _rows(1, k, 11)[0]
+    want, _ = _both(lin, x)
+    buf = hip.DeviceBuffer(8 * k)
+    for offset in (0, 16):  # words of x between its start and that of y
+        buf.upload(np.concatenate([x, np.zeros(k, np.float32)]))
+        lin.forward_dev(1, buf.ptr, buf.ptr + 4 * offset)
+        hip.check(hip.lib().syn_hip_stream_synchronize(None))
+        np.testing.assert_array_equal(buf.download(2 * k, np.uint32)[offset:offset + n], want)
+    buf.close()
+    lin.close()
