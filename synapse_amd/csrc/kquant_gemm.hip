@@ -958,8 +958,7 @@ static syn_status_t kq_gemm_f16(int fmt, bool exact, const u32x4 *W, const uint1
     // while it still reads x
     const bool can_split =
         ldy % 4 == 0 && reinterpret_cast<uintptr_t>(d_y) % 16 == 0 &&
-        !ranges_overlap(d_x, ((m - 1) * ldx + k) * sizeof(float), d_y,
-                        ((m - 1) * ldy + n) * sizeof(float));
+        !rows_overlap(d_x, m, k, ldx, d_y, n, ldy);
     const int kz = can_split ? rows_gemm_splits(g, m, false) : 1;
     SYN_TRY(ensure_rows(f16_rows_bytes(m, k), xh, xh_bytes));
     SYN_TRY(launch_rows_frag(fmt, d_x, ldx, m, k, false, xh.p, kz > 1 ? d_y : nullptr, ldy, n, s));
@@ -1005,9 +1004,11 @@ static syn_status_t kq_gemm_f16(int fmt, bool exact, const u32x4 *W, const uint1
   const int per = (int)cdiv((size_t)steps, (size_t)ksplit);
   ksplit = (int)cdiv((size_t)steps, (size_t)per);
   // a K split adds its partial tiles into Y: the conversion kernel clears Y
-  // (row-aligned 16-byte rows), else a kernel of its own does
+  // while it reads X (row-aligned 16-byte rows that do not overlap X), else a
+  // kernel of its own does after it
   const bool zero_in_conv =
-      ksplit > 1 && ldy % 4 == 0 && reinterpret_cast<uintptr_t>(d_y) % 16 == 0 && n < (1u << 31);
+      ksplit > 1 && ldy % 4 == 0 && reinterpret_cast<uintptr_t>(d_y) % 16 == 0 &&
+      n < (1u << 31) && !rows_overlap(d_x, m, k, ldx, d_y, n, ldy);
   float *rowmul = nullptr;
   SYN_TRY(to_f16_rows(m, k, d_x, ldx, xh, xh_bytes, false, &rowmul, s,
                       zero_in_conv ? d_y : nullptr, ldy, n));

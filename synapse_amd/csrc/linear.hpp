@@ -32,6 +32,12 @@ inline bool ranges_overlap(const void *a, size_t a_bytes, const void *b, size_t 
   const uintptr_t p = reinterpret_cast<uintptr_t>(a), q = reinterpret_cast<uintptr_t>(b);
   return p < q + b_bytes && q < p + a_bytes;
 }
+// x [m, k] (stride ldx) and y [m, n] (stride ldy) share memory
+inline bool rows_overlap(const float *x, size_t m, size_t k, size_t ldx, const float *y, size_t n,
+                         size_t ldy) {
+  return ranges_overlap(x, ((m - 1) * ldx + k) * sizeof(float), y,
+                        ((m - 1) * ldy + n) * sizeof(float));
+}
 
 // INT8 W8A8 linear: QuantizedLinear (quantization/primitives/int8_linear.rs)
 struct QLinearInt8 {

@@ -131,3 +131,24 @@ def test_wide_scales_keep_the_gemv(d):
     lin = hip.QLinear.q4_0(raw.reshape(-1), n, k)
     _check(lin, w, rng.standard_normal((m, k)).astype(np.float32), True)
     lin.close()
+
+
+# y over x, or over its upper part, where K splits add into rows that are cleared first: 24 rows
+# of the few-row kernel, 512 of the tiled one (two splits each on separate buffers)
+@pytest.mark.parametrize("m", [24, 512])
+@pytest.mark.parametrize("offset", [0, 64], ids=["same", "shifted"])
+def test_k_split_in_place(m, offset):
+    n = k = 4096
+    lin, w = _linear(hip.FMT_Q8_0, n, k, 4)
+    x = np.random.default_rng(m).standard_normal((m, k)).astype(np.float32)
+    buf = hip.DeviceBuffer(4 * (m * k + offset))
+    buf.upload(np.concatenate([x.ravel(), np.zeros(offset, np.float32)]))
+    lin.forward_dev(m, buf.ptr, buf.ptr + 4 * offset)
+    hip.check(hip.lib().syn_hip_stream_synchronize(None))
+    got = buf.download(m * k + offset, np.float32)[offset:].reshape(m, n).astype(np.float64)
+    size = np.abs(x).astype(np.float64) @ np.abs(w).T
+    worst = float((np.abs(got - x.astype(np.float64) @ w.T) / size).max())
+    print("m", m, "offset", offset, "worst", worst, flush=True)
+    assert worst <= 2.0**-10 * (1 + 2.0**-4)
+    buf.close()
+    lin.close()
