@@ -496,8 +496,12 @@ bool rows_gemm_fits(int fmt, bool q8_exact, size_t m, size_t n, size_t k) {
          (m <= 1024 && m * n * k <= 2200000000u);
 }
 
+// More than two f32 adds into a cleared element depend on their order; two do
+// not.  Where the tiled kernels take at most two K splits (128 tiles of 128 x
+// 128), so does this one, and the bits of such a call repeat
 int rows_gemm_splits(const RowsGemm &g, size_t m, bool split) {
-  return shape_of(g, m, kRowsMaxSplit, split).kz;
+  const bool repeats = !split && cdiv(g.n, 128) * cdiv(m, 128) >= 128;
+  return shape_of(g, m, repeats ? 2 : kRowsMaxSplit, split).kz;
 }
 
 syn_status_t launch_rows_frag(int fmt, const float *x, size_t ldx, size_t m, size_t k, bool split,

@@ -152,3 +152,31 @@ def test_k_split_in_place(m, offset):
     assert worst <= 2.0**-10 * (1 + 2.0**-4)
     buf.close()
     lin.close()
+
+
+def _raw(fmt, n, k, seed):
+    """a handle over random bytes with scales of about 0.01"""
+    size, at = {hip.FMT_Q4_0: (18, (0,)), hip.FMT_Q8_0: (34, (0,)), hip.FMT_Q4_K: (144, (0, 2)),
+                hip.FMT_Q6_K: (210, (208,))}[fmt]
+    rng = np.random.default_rng(seed)
+    raw = rng.integers(0, 256, (n * k // EL[fmt], size), dtype=np.uint8)
+    d = (rng.random(len(raw)) * 0.01 + 0.005).astype(np.float16).view(np.uint8).reshape(-1, 2)
+    for a in at:
+        raw[:, a:a + 2] = d
+    if fmt == hip.FMT_Q4_0:
+        return hip.QLinear.q4_0(raw.reshape(-1), n, k)
+    return hip.QLinear.gguf(fmt, raw.reshape(-1), n, k)
+
+
+# shapes whose least time by the launch rule's count is at three or four K splits, on grids where
+# at most two are taken: the same bits from call to call
+@pytest.mark.parametrize("fmt,m,n,k", [(hip.FMT_Q8_0, 15, 20040, 9216),
+                                       (hip.FMT_Q4_K, 26, 17000, 10752),
+                                       (hip.FMT_Q6_K, 9, 16388, 14336)])
+def test_bits_repeat(fmt, m, n, k):
+    lin = _raw(fmt, n, k, m)
+    x = np.random.default_rng(k).standard_normal((m, k)).astype(np.float32)
+    first = lin.forward(x).view(np.uint32)
+    for _ in range(6):
+        np.testing.assert_array_equal(lin.forward(x).view(np.uint32), first)
+    lin.close()
