@@ -481,19 +481,39 @@ size_t rows_frag_bytes(size_t m, size_t k, bool split) {
 }
 
 // Where the line to the tiled kernels lies (whole calls, us, here against
-// tiled).  Up to 128 rows always: 14336 -> 4096 x 64 rows Q8_0 24 against 42,
-// 2048 -> 16384 x 128 24 against 30, 4096 -> 14336 x 128 34 against 42 (192
-// rows 49 against 52, Q4_K 56 against 59; 256 rows 64 against 56).  To 256
-// rows for n <= 8192: 3072 -> 8192 30 against 34, 14336 -> 4096 51 against
-// 56 (2048 -> 16384 43 against 31).  To 512 rows while m n <= 1.6e6: 14336
-// -> 4096 x 384 88 against 99, 8192 -> 2048 x 512 36 against 41 (14336 ->
-// 4096 x 512 97 against 90, 3072 -> 8192 x 512 49 against 39).  To 1024 rows
-// while m n k <= 2.2e9: 1024 -> 2048 x 1024 20 against 27, 2048 -> 1024 x
-// 1024 18 against 27 (14336 -> 1024 x 768 73 against 58).
+// tiled).
+//  - Up to 64 rows always: 14336 -> 4096 x 64 rows Q8_0 24 against 42; Q4_K 3072
+//    -> 32000 39 against 68, Q6_K 3072 -> 128256 149 against 250.
+//  - Up to 128 rows, each 64 of which decode the weights again: 4096 -> 14336 x
+//    128 34 against 42, Q4_K 3072 -> 32000 67 against 69.  Not on a short K
+//    where the tiled kernel's columns of 128 fill one or two rounds of 256 CUs
+//    (128 rows, 1024 -> 32768 Q8_0 31 against 28, Q4_K 34 against 30, 1024 ->
+//    28672 Q4_K 0.85 times as fast, 1536 -> 32768 0.94, 2048 -> 30720 0.98, 1024
+//    -> 24576 and 49152, where the last round is half empty, 1.1 to 1.2; Q4_0
+//    0.97 and more everywhere).
+//  - To 256 rows for n <= 8192: 3072 -> 8192 30 against 34, 14336 -> 4096 52
+//    against 57, 14336 -> 7168 1.07 to 1.5 times as fast (2048 -> 16384 43 against
+//    31).  At n = 8192 the tiled kernel's two K splits fill 256 CUs: 14336 -> 8192 x
+//    192 Q8_0 100 against 86, 256 Q4_K 114 against 100 (Q4_0 84 against 87).
+//  - To 512 rows while m n <= 1.6e6: 14336 -> 4096 x 384 88 against 99, 8192 ->
+//    2048 x 512 36 against 41 (14336 -> 4096 x 512 97 against 90, 3072 -> 8192 x
+//    512 49 against 39).
+//  - To 1024 rows while m n k <= 2.2e9: 1024 -> 2048 x 1024 20 against 27, 2048 ->
+//    1024 x 1024 18 against 27 (14336 -> 1024 x 768 73 against 58); for Q8_0, whose
+//    tiled kernel is the fastest, 1.5e9 at K of 4096 to 8192 (8192 -> 256 x 1024
+//    40 against 36, x 768 32 against 33).
 bool rows_gemm_fits(int fmt, bool q8_exact, size_t m, size_t n, size_t k) {
   if (fmt == SYN_HIP_FMT_Q8_0 && !q8_exact) return false;
-  return m <= 128 || (m <= 256 && n <= 8192) || (m <= 512 && m * n <= 1600000) ||
-         (m <= 1024 && m * n * k <= 2200000000u);
+  if (m <= 64) return true;
+  if (m <= 128) {
+    const size_t tiles = cdiv(n, 128), rounds = cdiv(tiles, 256);
+    const bool full = rounds <= 2 && 8 * tiles >= 7 * 256 * rounds;
+    return fmt == SYN_HIP_FMT_Q4_0 || !full || k > 1536;
+  }
+  if (m <= 256 && n <= 8192) return fmt == SYN_HIP_FMT_Q4_0 || n <= 7168 || k < 8192;
+  if (m <= 512 && m * n <= 1600000) return true;
+  const bool tiled_q8 = fmt == SYN_HIP_FMT_Q8_0 && k > 4096 && k <= 8192;
+  return m <= 1024 && m * n * k <= (tiled_q8 ? 1500000000u : 2200000000u);
 }
 
 // More than two f32 adds into a cleared element depend on their order; two do

@@ -155,7 +155,7 @@ def test_k_split_in_place(m, offset):
 
 
 def _raw(fmt, n, k, seed):
-    """a handle over random bytes with scales of about 0.01"""
+    """a handle over random bytes with scales of about 0.01, and the bytes"""
     size, at = {hip.FMT_Q4_0: (18, (0,)), hip.FMT_Q8_0: (34, (0,)), hip.FMT_Q4_K: (144, (0, 2)),
                 hip.FMT_Q6_K: (210, (208,))}[fmt]
     rng = np.random.default_rng(seed)
@@ -164,8 +164,8 @@ def _raw(fmt, n, k, seed):
     for a in at:
         raw[:, a:a + 2] = d
     if fmt == hip.FMT_Q4_0:
-        return hip.QLinear.q4_0(raw.reshape(-1), n, k)
-    return hip.QLinear.gguf(fmt, raw.reshape(-1), n, k)
+        return hip.QLinear.q4_0(raw.reshape(-1), n, k), raw
+    return hip.QLinear.gguf(fmt, raw.reshape(-1), n, k), raw
 
 
 # shapes whose least time by the launch rule's count is at three or four K splits, on grids where
@@ -174,9 +174,33 @@ def _raw(fmt, n, k, seed):
                                        (hip.FMT_Q4_K, 26, 17000, 10752),
                                        (hip.FMT_Q6_K, 9, 16388, 14336)])
 def test_bits_repeat(fmt, m, n, k):
-    lin = _raw(fmt, n, k, m)
+    lin, _ = _raw(fmt, n, k, m)
     x = np.random.default_rng(k).standard_normal((m, k)).astype(np.float32)
     first = lin.forward(x).view(np.uint32)
     for _ in range(6):
         np.testing.assert_array_equal(lin.forward(x).view(np.uint32), first)
+    lin.close()
+
+
+# both sides of the lines to the tiled kernels: 128 rows on full and part rounds of columns and at
+# K of 1536, the columns of 129 to 256 rows, the products m n and m n k, 512 and 1024 rows
+@pytest.mark.parametrize("fmt,n,k,rows", [
+    (hip.FMT_Q8_0, 28548, 256, (64, 65, 128)), (hip.FMT_Q4_K, 28676, 256, (64, 65, 128)),
+    (hip.FMT_Q6_K, 28676, 1792, (65, 128)), (hip.FMT_Q8_0, 28676, 1536, (128,)),
+    (hip.FMT_Q8_0, 7168, 8192, (129, 256)), (hip.FMT_Q8_0, 7172, 8192, (129, 256)),
+    (hip.FMT_Q4_K, 8196, 512, (128, 129)), (hip.FMT_Q4_0, 3128, 512, (511, 512)),
+    (hip.FMT_Q8_0, 256, 4128, (1024, 1025)), (hip.FMT_Q8_0, 256, 6144, (953, 954)),
+    (hip.FMT_Q6_K, 64, 512, (512, 513, 1024, 1025)), (hip.FMT_Q4_K, 260, 8192, (1024,))])
+def test_dispatch_lines(fmt, n, k, rows):
+    lin, raw = _raw(fmt, n, k, n)
+    if fmt == hip.FMT_Q4_0:
+        q = np.empty((len(raw), 32), np.float32)
+        q[:, 0::2], q[:, 1::2] = raw[:, 2:] & 15, raw[:, 2:] >> 4
+        w = (q - 8) * raw[:, :2].copy().view(np.float16).astype(np.float32)
+    else:
+        w = hip.kquant_decode(fmt, raw.reshape(-1))
+    w = w.astype(np.float64).reshape(n, k)
+    x = np.random.default_rng(k).standard_normal((max(rows), k)).astype(np.float32)
+    for m in rows:
+        _check(lin, w, x[:m], False)
     lin.close()
