@@ -167,7 +167,12 @@ syn_status_t syn_hip_qlinear_create(int fmt, size_t n, size_t k, const void *hos
 syn_status_t syn_hip_qlinear_from_f32(int fmt, size_t n, size_t k, const float *host_w,
                                       syn_hip_qlinear_t **out);
 /* y[m,n] = x[m,k] W^T.  INT8 quantizes x per row first (forward,
- * int8_linear.rs:87-117); Q4_0 runs f32 activations (Q4Linear::forward). */
+ * int8_linear.rs:87-117); Q4_0 runs f32 activations (Q4Linear::forward).
+ * A handle keeps scratch of its own (quantized rows, 16-bit rows, K-split
+ * sums), allocated by the first call that needs it: such a call cannot be the
+ * first one under graph capture, and calls on one handle that overlap
+ * (different streams or host threads) race on it.  Q4_0 rows of m <= 16 use
+ * none when n > 15296. */
 syn_status_t syn_hip_qlinear_forward(syn_hip_qlinear_t *h, size_t m, const float *d_x,
                                      float *d_y, void *stream);
 /* No counterpart in the reference: syn_hip_qlinear_forward for INT8 handles

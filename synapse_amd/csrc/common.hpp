@@ -127,6 +127,20 @@ __device__ __forceinline__ float kqf_unfix(long long a) {
 // clang vector types (usable with __builtin_nontemporal_load)
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// 4 x 4 transpose between the four groups of 16 lanes and the elements of v:
+// element g of group s goes to element s of group g
+__device__ __forceinline__ f32x4 groups_transposed(f32x4 v) {
+  const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v.x), __float_as_uint(v.z),
+                                                  false, false);
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v.y), __float_as_uint(v.w),
+                                                  false, false);
+  const auto c = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);
+  const auto d = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+  return f32x4{__uint_as_float(c[0]), __uint_as_float(c[1]), __uint_as_float(d[0]),
+               __uint_as_float(d[1])};
+}
 
 // T[i] = asuint64(2^(i/32)) - (i << 47)
 static __constant__ uint64_t syn_exp2_tab[32] = {

@@ -18,7 +18,6 @@ namespace syn {
 
 namespace {
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 enum { HEAD_FX = 0, HEAD_ACC = 1, HEAD_F32 = 2 };
 

@@ -671,7 +671,7 @@ syn_status_t syn_hip_qlinear_forward_noalloc(syn_hip_qlinear_t *h, size_t m, con
                                              float *d_y, void *stream) {
   if (!h) return SYN_ERR_NULL_PTR;
   if (h->fmt != SYN_HIP_FMT_INT8) {
-    set_error("qlinear_forward_noalloc: INT8 handles only (the other formats use no scratch)");
+    set_error("qlinear_forward_noalloc: INT8 handles only");
     return SYN_ERR_INVALID_ARG;
   }
   if (m == 0) return SYN_OK;

@@ -25,7 +25,6 @@
 namespace syn {
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // x f32 [M, ldx] -> xh f16 [M, ldh], columns K..ldh-1 zero (K a multiple of
 // 8, ldh of 64, ldx of 4), one workgroup per row.  Each row is scaled by a

@@ -467,19 +467,6 @@ __host__ __device__ __forceinline__ int pf_ld(int t) {
   return (w + 59) / 64 * 64 + 4;
 }
 
-// 4 x 4 transpose between the four groups of 16 lanes and the elements of v:
-// element g of group s goes to element s of group g
-__device__ __forceinline__ f32x4 groups_transposed(f32x4 v) {
-  const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v.x), __float_as_uint(v.z),
-                                                  false, false);
-  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v.y), __float_as_uint(v.w),
-                                                  false, false);
-  const auto c = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);
-  const auto d = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
-  return f32x4{__uint_as_float(c[0]), __uint_as_float(c[1]), __uint_as_float(d[0]),
-               __uint_as_float(d[1])};
-}
-
 template <int HD, bool EXACT>
 __global__ void __launch_bounds__(kPfThreads)
     k_attn_prefill_mfma(const float *__restrict__ q, const float *__restrict__ kc,

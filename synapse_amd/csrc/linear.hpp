@@ -129,7 +129,7 @@ struct QLinearQ4_0 {
   bool has_wide_scale = false;  // 8 d is beyond f16 for some block scale d, or d is not finite
   DevBuf xh;                         // f16 activations for the MFMA GEMM
   size_t xh_bytes = 0;  // its size (f16_rows_bytes)
-  SplitKSlots sk;  // gemv()'s one-launch K split at one row (split_k.hpp)
+  SplitKSlots sk;  // gemv()'s one-launch K split (split_k.hpp)
   syn_status_t upload_packed(const uint8_t *packed, size_t n_, size_t k_);
   syn_status_t from_f32(const float *w_nk, size_t n_, size_t k_);
   // allocate the split-K partials of GEMV batches up to max_m rows (so that
@@ -147,10 +147,10 @@ struct QLinearQ4_0 {
   // activations rounded once to f16, f32 accumulation
   syn_status_t gemm(size_t m, const float *d_x, size_t ldx, float *d_y, size_t ldy,
                     hipStream_t s);
-  // 7 to 16 rows on the matrix cores with f32 accuracy (rows_gemm.hip)
-  syn_status_t gemm_split(size_t m, const float *d_x, size_t ldx, float *d_y, size_t ldy,
-                          hipStream_t s);
-  syn_status_t ensure_split(size_t m);
+  // up to 16 rows on the matrix cores, operands unrounded
+  syn_status_t rows16(size_t m, const float *d_x, size_t ldx, float *d_y, size_t ldy,
+                      hipStream_t s);
+  syn_status_t ensure_slots();
   // the GEMM decodes the scales as IEEE f16 values: not for halved subnormals
   bool gemm_ok() const { return !(rs_f16_scales && has_subnormal_scale); }
   // the split form also needs (nibble - 8) * d within f16's range

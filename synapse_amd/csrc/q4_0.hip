@@ -13,8 +13,8 @@
 #include <cmath>
 #include <vector>
 
+#include "bf16_parts.hpp"
 #include "linear.hpp"
-#include "rows_gemm.hpp"
 #include "split_k.hpp"
 
 namespace syn {
@@ -309,6 +309,185 @@ __global__ void __launch_bounds__(512)
   }
 }
 
+// Up to 16 rows on the matrix cores.  A GEMV launch takes eight rows, reads the
+// weights once per launch and spends 32 FMAs a block, row and column; here a
+// wave forms 16 rows x 16 columns of a block's dots with three MFMAs.  Every
+// operand is exact (bf16_parts.hpp): the activations as three bf16, the levels
+// as one, the products in f32; a block's dot is scaled in f32 afterwards, as
+// in the GEMV.  No scratch: a wave reads the f32 rows itself, lane (g, r) =
+// (lane / 16, lane % 16) the elements 8g .. 8g+7 of row r and, of column r,
+// block g of the step's four, whose dwords a transpose between the groups
+// hands to the lanes that hold their elements.  A sum that is not finite (an
+// infinity or a NaN, or activations beyond the parts' range) is formed again
+// from the weights' values in plain f32.
+// grid (columns / 16 NT, K splits); the eight waves take the slice's steps of
+// four blocks in turn, two steps in flight.  A K split finishes in the same
+// launch, in slice order (split_k.hpp).  Bound by each workgroup's pass over the
+// rows of x, from L2, and the latency of its two or three steps (16 rows, 3072
+// -> 8192: 12.8 us for 14 MB of weights; 12 rows 12.0, 7 rows 10.7).  Sixteen
+// waves measured up to 12 % slower, and loads of 64 whole bytes a row the same.
+constexpr int kRows16 = 16, kRows16Waves = 8;
+
+template <int NT>
+__global__ void __launch_bounds__(64 * kRows16Waves)
+    k_rows16_q4_0(const u32x4 *__restrict__ nib, const uint16_t *__restrict__ sc,
+                  const float *__restrict__ x, int ldx, int M, float *__restrict__ y, int ldy,
+                  unsigned *__restrict__ skacc, int *__restrict__ skcnt, int N, int B, int per,
+                  float sub) {
+  constexpr int NW = kRows16Waves, CP = 16 * NT + 4;
+  __shared__ float red[NW][kRows16][CP];
+  __shared__ int s_last;
+  const int tid = threadIdx.x, lane = tid & 63, c16 = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n0 = blockIdx.x * 16 * NT, steps = (B + 3) >> 2;
+  const int s0 = blockIdx.y * per, s1 = min(steps, s0 + per);
+  const float *xr = x + (size_t)min(c16, M - 1) * ldx + 8 * g;
+  const int last = ((N + 63) >> 6) * 64 - 1;  // the last panel's padding rows are not stored
+  size_t at[NT];
+#pragma unroll
+  for (int t = 0; t < NT; t++) {
+    const int n = min(n0 + 16 * t + c16, last);
+    at[t] = (size_t)(n >> 6) * B * 64 + (n & 63);
+  }
+  struct Step {
+    float4 x[4][2];
+    u32x4 q[NT];
+    uint16_t d[NT];
+  };
+  auto load = [&](Step &st, int step) {  // past the last block: the last one again
+    const size_t b = (size_t)min(4 * step + g, B - 1) * 64;
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+      st.q[t] = __builtin_nontemporal_load(nib + at[t] + b);
+      st.d[t] = __builtin_nontemporal_load(sc + at[t] + b);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const float4 *p = reinterpret_cast<const float4 *>(xr + (size_t)min(4 * step + j, B - 1) * 32);
+      st.x[j][0] = p[0];
+      st.x[j][1] = p[1];
+    }
+  };
+  f32x4 acc[NT];
+#pragma unroll
+  for (int t = 0; t < NT; t++) acc[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  auto mul = [&](const Step &st, int step) {
+    f32x4 q[NT], d[NT];  // element j: of block j of the step
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+      q[t] = groups_transposed(__builtin_bit_cast(f32x4, st.q[t]));
+      const float s = q4_scale(st.d[t], sub);
+      d[t] = groups_transposed(f32x4{s, s, s, s});
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      if (4 * step + j >= B) break;
+      const float4 a = st.x[j][0], b = st.x[j][1];
+      const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+      bf16x8 p[3];
+      bf16_parts(v, p);
+#pragma unroll
+      for (int t = 0; t < NT; t++) {
+        const bf16x8 w = q4_levels(__float_as_uint(q[t][j]));
+        f32x4 dot = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int i = 2; i >= 0; i--)
+          dot = __builtin_amdgcn_mfma_f32_16x16x32_bf16(p[i], w, dot, 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < 4; r++) acc[t][r] = __builtin_fmaf(dot[r], d[t][j], acc[t][r]);
+      }
+    }
+  };
+  auto hold = [] { __builtin_amdgcn_sched_barrier(0); };  // as in k_rows_gemm
+  Step st0, st1;
+  int step = s0 + wave;
+  if (step < s1) {
+    load(st0, step); hold();
+    load(st1, min(step + NW, s1 - 1)); hold();
+    while (true) {
+      mul(st0, step);
+      step += NW;
+      if (step >= s1) break;
+      load(st0, min(step + NW, s1 - 1)); hold();
+      mul(st1, step);
+      step += NW;
+      if (step >= s1) break;
+      load(st1, min(step + NW, s1 - 1)); hold();
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < NT; t++)
+#pragma unroll
+    for (int r = 0; r < 4; r++) red[wave][4 * g + r][16 * t + c16] = acc[t][r];
+  __syncthreads();
+  const int N64 = (last + 1), S = gridDim.y;
+  auto sum = [&](int r, int c) {
+    float v = 0.0f;
+#pragma unroll
+    for (int w = 0; w < NW; w++) v += red[w][r][c];
+    if (fabsf(v) <= 3.4028235e38f) return v * kPartsDown;
+    const int n = n0 + c;
+    const float *xp = x + (size_t)r * ldx;
+    v = 0.0f;
+    for (int b = 4 * s0; b < min(B, 4 * s1); b++) {
+      const size_t i = ((size_t)(n >> 6) * B + b) * 64 + (n & 63);
+      const u32x4 q = nib[i];
+      const float d = q4_scale(sc[i], sub);
+      for (int e = 0; e < 32; e++) {
+        const uint32_t w = e < 8 ? q.x : e < 16 ? q.y : e < 24 ? q.z : q.w;
+        const float level = (float)((w >> (4 * (e & 7))) & 15u) - 8.0f;
+        v = __builtin_fmaf(xp[b * 32 + e], level * d, v);
+      }
+    }
+    return v;
+  };
+  constexpr int E = kRows16 * 16 * NT, NTHR = 64 * NW;
+  if (S == 1) {
+    for (int i = tid; i < E; i += NTHR) {
+      const int r = i / (16 * NT), c = i % (16 * NT);
+      if (r < M && n0 + c < N) y[(size_t)r * ldy + n0 + c] = sum(r, c);
+    }
+    return;
+  }
+  unsigned seen = 0;
+  for (int i = tid; i < E; i += NTHR) {
+    const int r = i / (16 * NT), c = i % (16 * NT);
+    if (r < M && n0 + c < N)
+      seen |= sk_put(skacc + ((size_t)r * S + blockIdx.y) * N64 + n0 + c, sum(r, c));
+  }
+  int *cnt = skcnt + blockIdx.x;
+  if (!sk_arrive(seen, cnt, S, &s_last)) return;
+  for (int i = tid; i < E; i += NTHR) {
+    const int r = i / (16 * NT), c = i % (16 * NT);
+    if (r < M && n0 + c < N)
+      y[(size_t)r * ldy + n0 + c] = sk_sum(skacc + (size_t)r * S * N64 + n0 + c, N64, S);
+  }
+  sk_reset(cnt);
+}
+
+// Columns per workgroup (16 nt) and K splits of a k_rows16_q4_0 launch: 32
+// columns while that is one round of workgroups on 256 CUs, else 64, which read
+// the activations half as often (16 rows, us: 2048 -> 8192 9.8 against 13.0,
+// 4096 -> 11008 24.6 against 20.8); K splits up to one round, each of half a
+// step or more for every wave (4096 -> 1024 in eight 7.5, in four 8.8, unsplit
+// 14.3; 14336 -> 512 in sixteen 10.8, in eight 11.9).  K is split only where the
+// GEMV's is: other grids need no slots, and no call of theirs allocates.
+struct Rows16Plan {
+  int nt, tiles, ks, per;
+};
+static Rows16Plan rows16_plan(size_t n, int blocks) {
+  Rows16Plan o;
+  const int steps = (blocks + 3) / 4;
+  o.nt = n <= 8192 ? 2 : 4;
+  o.tiles = (int)cdiv(n, (size_t)(16 * o.nt));
+  o.ks = 1;
+  if (make_gemv_plan(n, (size_t)blocks, false).ksplit > 1)
+    o.ks = std::max(1, std::min(256 / o.tiles, 2 * steps / kRows16Waves));
+  o.per = (int)cdiv((size_t)steps, (size_t)o.ks);
+  o.ks = (int)cdiv((size_t)steps, (size_t)o.per);
+  return o;
+}
+
 // U blocks in flight per wave: 8 with 8 waves when a slice has >= 64
 // blocks (four workgroups per CU stream the matrix), else 4 with up to 16
 template <int M>
@@ -338,18 +517,19 @@ syn_status_t QLinearQ4_0::gemv(size_t m, const float *d_x, size_t ldx, float *d_
                                hipStream_t s) {
   if (m == 0 || n == 0 || k == 0) return SYN_OK;
   if (m > 16 && gemm_ok() && ldx % 4 == 0) return gemm(m, d_x, ldx, d_y, ldy, s);
-  // 9 to 16 rows: two GEMV launches read the weights twice (3072 -> 8192: 25-37
-  // us against 12 on the matrix cores, 4096 -> 1024 16-18 against 12.5, 2048
-  // -> 2048 13-15 against 9).  7 and 8 rows only on large matrices (8 rows,
-  // 3072 -> 8192 18.6 against 12, 14336 -> 4096 38 against 30; 4096 -> 1024
-  // 9.0 against 12.5)
-  if (split_ok() && ldx % 4 == 0 && m <= 16 && (m >= 9 || (m >= 7 && n * k >= 24000000)))
-    return gemm_split(m, d_x, ldx, d_y, ldy, s);
+  // 9 to 16 rows: two GEMV launches read the weights twice (12 rows, us: 3072 ->
+  // 8192 30.3 against 12.0 here, 4096 -> 1024 16.8 against 7.2, 14336 -> 512 21.2
+  // against 10.1, 2048 -> 16384 35.5 against 13.1, 512 -> 256 13.1 against 4.6).  7
+  // and 8 rows from 24e6 weights on (8 rows, 3072 -> 8192 19.7 against 11.0, 14336
+  // -> 2048 21.7 against 13.8); below, the GEMV's one launch stays, though only 8
+  // rows of 512 -> 32768 measured faster there (9.3 against 10.2)
+  if (m <= 16 && ldx % 4 == 0 && (m >= 9 || (m >= 7 && n * k >= 24000000)))
+    return rows16(m, d_x, ldx, d_y, ldy, s);
   const float sub = rs_f16_scales ? 0.5f : 1.0f;
   // "chunks" here are 32-element blocks; a K slice holds whole blocks.  One
   // launch per block of up to 8 rows: a K split finishes in place (split_k.hpp)
   const GemvPlan p = make_gemv_plan(n, (size_t)blocks, false);
-  if (p.ksplit > 1) SYN_TRY(sk.ensure(p.panels, 8, p.ksplit));
+  SYN_TRY(ensure_slots());
   for (size_t m0 = 0; m0 < m; m0 += 8) {
     const int mb = (int)std::min<size_t>(8, m - m0);
     const size_t shm_h = ((size_t)p.cs + 8 * 64) * 4;
@@ -368,27 +548,23 @@ syn_status_t QLinearQ4_0::gemv(size_t m, const float *d_x, size_t ldx, float *d_
   return SYN_OK;
 }
 
-syn_status_t QLinearQ4_0::gemm_split(size_t m, const float *d_x, size_t ldx, float *d_y,
-                                     size_t ldy, hipStream_t s) {
-  RowsGemm g;
-  g.fmt = SYN_HIP_FMT_Q4_0;
-  g.W = nib.p;
-  g.Wd = sc.as<uint16_t>();
-  g.blocks = blocks;
-  g.n = n;
-  g.k = k;
-  SYN_TRY(ensure_split(m));
-  SYN_TRY(launch_rows_frag(g.fmt, d_x, ldx, m, k, true, xh.p, nullptr, 0, 0, s));
-  return launch_rows_gemm_split(g, xh.p, m, 1, d_y, ldy, 0, s);
+syn_status_t QLinearQ4_0::rows16(size_t m, const float *d_x, size_t ldx, float *d_y, size_t ldy,
+                                 hipStream_t s) {
+  SYN_TRY(ensure_slots());
+  const Rows16Plan o = rows16_plan(n, blocks);
+  const auto kern = o.nt == 2 ? k_rows16_q4_0<2> : k_rows16_q4_0<4>;
+  hipLaunchKernelGGL(kern, dim3(o.tiles, o.ks), dim3(64 * kRows16Waves), 0, s, nib.as<u32x4>(),
+                     sc.as<uint16_t>(), d_x, (int)ldx, (int)m, d_y, (int)ldy, sk.slots(),
+                     sk.counters(), (int)n, blocks, o.per, rs_f16_scales ? 0.5f : 1.0f);
+  SYN_LAUNCH_CHECK();
+  return SYN_OK;
 }
 
-syn_status_t QLinearQ4_0::ensure_split(size_t m) {
-  const size_t need = rows_frag_bytes(m, k, true);
-  if (xh_bytes >= need) return SYN_OK;
-  SYN_HIP(hipDeviceSynchronize());  // the old buffer may still be read by queued work
-  SYN_TRY(xh.alloc(need));
-  xh_bytes = need;
-  return SYN_OK;
+// slots for every gemv() of up to 16 rows at once: none is reallocated later
+syn_status_t QLinearQ4_0::ensure_slots() {
+  const GemvPlan p = make_gemv_plan(n, (size_t)blocks, false);
+  if (p.ksplit <= 1) return SYN_OK;
+  return sk.ensure(p.panels, kRows16, std::max(p.ksplit, rows16_plan(n, blocks).ks));
 }
 
 syn_status_t QLinearQ4_0::gemv_parts(const float *d_x, float *d_y, PartRows *out,
@@ -414,8 +590,7 @@ syn_status_t QLinearQ4_0::gemv_parts(const float *d_x, float *d_y, PartRows *out
 
 syn_status_t QLinearQ4_0::prepare(size_t max_m) {
   const GemvPlan p = make_gemv_plan(n, (size_t)blocks, false);
-  if (p.ksplit > 1) SYN_TRY(sk.ensure(p.panels, 8, p.ksplit));
-  if (max_m >= 7) SYN_TRY(ensure_split(std::min<size_t>(16, max_m)));
+  SYN_TRY(ensure_slots());
   const size_t need = (size_t)p.ksplit * std::min<size_t>(8, max_m) * (size_t)p.panels * 64;
   if (p.ksplit > 1 && part_elems < need) {
     part_elems = need;

@@ -13,7 +13,6 @@ __device__ __forceinline__ void bar() {
   else __builtin_amdgcn_wave_barrier();
 }
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // Makes the registers of `a` an input and output of an empty asm statement:
 // every load that produces them completes before this point, and no

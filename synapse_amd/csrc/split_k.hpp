@@ -91,7 +91,8 @@ __device__ __forceinline__ bool sk_slots_last(float v, unsigned *slots, size_t s
   return true;
 }
 
-// The slots [rows][slices][panels * 64] and counters [panels] of one handle.
+// The slots [rows][slices][panels * 64] and counters (four a panel: a tile may
+// be 16 columns) of one handle.
 // Counters are zero between calls (allocated and cleared once, outside any
 // graph capture); slots are written before they are read in every call.
 struct SplitKSlots {
@@ -104,7 +105,7 @@ struct SplitKSlots {
     slices_ = std::max(slices_, slices);
     SYN_HIP(hipDeviceSynchronize());  // the old buffers may still be in use by queued work
     SYN_TRY(part.alloc((size_t)rows_ * slices_ * panels_ * 64 * sizeof(unsigned)));
-    SYN_TRY(cnt.alloc((size_t)panels_ * sizeof(int)));
+    SYN_TRY(cnt.alloc((size_t)panels_ * 4 * sizeof(int)));
     SYN_HIP(hipMemset(cnt.p, 0, cnt.bytes));
     SYN_HIP(hipDeviceSynchronize());  // the memset runs on the null stream, not the caller's
     panels = panels_;

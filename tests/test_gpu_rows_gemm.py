@@ -3,11 +3,11 @@ weights, at the edges of its tiles and of its dispatch rule.
 
 Bounds, per element and relative to sum |x w|: one f16 rounding (2^-11) of
 each activation and each weight, plus f32 sums, stay below 2^-10 (1 + 2^-4).
-Split Q4_0 (7 to 16 rows): the weights are exact, an activation's two halves
-leave at most 2^-22 of it, the product of the remainders that is not formed
-2^-22, and the f32 sums of at most K / 16 + 16 partial sums 2^-24 each."""
+Q4_0 at 7 to 16 rows: activations, levels and products are exact, and what is
+left is the f32 sums, of fewer than K / 16 + 24 partial sums 2^-24 each."""
 import numpy as np
 import pytest
+import torch
 
 from synapse_amd import hip
 
@@ -79,7 +79,7 @@ def test_rows_gemm_half_step_tail(fmt, k):
 
 
 def test_split_rows_seven_and_eight():
-    # 7 and 8 rows take the split form from 24e6 weights on; both sides of the line
+    # 7 and 8 rows take the matrix cores from 24e6 weights on; both sides of the line
     for n, k in ((8192, 3072), (1024, 2048)):
         lin, w = _linear(hip.FMT_Q4_0, n, k, 3)
         x = np.random.default_rng(5).standard_normal((8, k)).astype(np.float32)
@@ -117,7 +117,7 @@ def test_split_rows_extremes():
 
 @pytest.mark.parametrize("d", [2.0**13, 65504.0])
 def test_wide_scales_keep_the_gemv(d):
-    # 8 d beyond f16: the rows stay on the f32 GEMV
+    # 8 d beyond f16: the levels are scaled in f32
     n, k, m = 64, 512, 12
     rng = np.random.default_rng(21)
     raw = rng.integers(0, 256, (n * k // 32, 18), dtype=np.uint8)
@@ -203,4 +203,96 @@ def test_dispatch_lines(fmt, n, k, rows):
     x = np.random.default_rng(k).standard_normal((max(rows), k)).astype(np.float32)
     for m in rows:
         _check(lin, w, x[:m], False)
+    lin.close()
+
+
+def _q4_0(n, k, d, seed):
+    """a Q4_0 handle's bytes with the block scales d, and its float64 weights"""
+    raw = np.random.default_rng(seed).integers(0, 256, (n * k // 32, 18), dtype=np.uint8)
+    raw[:, :2] = d.view(np.uint8).reshape(-1, 2)
+    q = np.empty((len(raw), 32))
+    q[:, 0::2], q[:, 1::2] = raw[:, 2:] & 15, raw[:, 2:] >> 4
+    return raw, ((q - 8) * d.astype(np.float64)[:, None]).reshape(n, k)
+
+
+# an activation 2^30 times the others, on weights of zero: the others keep all of their bits
+@pytest.mark.parametrize("k", [64, 2048])
+def test_q4_0_rows_beside_an_outlier(k):
+    n, m = 96, 12
+    rng = np.random.default_rng(k)
+    raw, w = _q4_0(n, k, (rng.random(n * k // 32) * 0.01 + 1e-3).astype(np.float16), k)
+    raw.reshape(n, -1, 18)[:, 1, 2 + 3] = 0x88  # elements 6 and 7 of every row's second block
+    w[:, 32 + 6:32 + 8] = 0
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    x[:, 32 + 6] = 2.0**30
+    lin = hip.QLinear.q4_0(raw.reshape(-1), n, k)
+    _check(lin, w, x, True)
+    lin.close()
+
+
+# subnormal block scales, as IEEE values and (GGUF) halved, in the K split and without it
+@pytest.mark.parametrize("gguf", [False, True])
+@pytest.mark.parametrize("m", [9, 16])
+def test_q4_0_rows_subnormal_scales(m, gguf):
+    n, k = 72, 1056
+    rng = np.random.default_rng(m)
+    d = (rng.random(n * k // 32) * 0.01 + 1e-3).astype(np.float16)
+    d[::3] = rng.integers(1, 1024, len(d[::3]), dtype=np.uint16).view(np.float16)
+    raw, w = _q4_0(n, k, d, m)
+    if gguf:
+        w.reshape(-1, 32)[::3] *= 0.5
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    x[:, 96:128] *= 1e4  # a block whose scale is subnormal counts
+    lin = hip.QLinear.q4_0(raw.reshape(-1), n, k, gguf_dequant=gguf)
+    _check(lin, w, x, True)
+    lin.close()
+
+
+# columns of 32 and 64 a workgroup (the line at 8192) with parts of the last one, block counts that
+# are no whole steps of four, K splits
+@pytest.mark.parametrize("n,k", [(8196, 288), (8192, 96), (8188, 1056), (16404, 160), (1000, 14336),
+                                 (40, 2112), (15300, 64)])
+def test_q4_0_rows_columns(n, k):
+    rng = np.random.default_rng(n)
+    raw, w = _q4_0(n, k, (rng.random(n * k // 32) * 0.01 + 1e-3).astype(np.float16), n)
+    x = rng.standard_normal((16, k)).astype(np.float32)
+    x[0, 5], x[3, 7], x[4, 8] = np.inf, 1e38, np.nan
+    lin = hip.QLinear.q4_0(raw.reshape(-1), n, k)
+    for m in (9, 16):
+        got = lin.forward(x[:m]).astype(np.float64)
+        assert np.isnan(got[4]).all() and not np.isfinite(got[0]).any()
+        rows = [r for r in range(m) if r not in (0, 4)]
+        size = np.abs(x[rows]).astype(np.float64) @ np.abs(w).T
+        worst = float((np.abs(got[rows] - x[rows].astype(np.float64) @ w.T) / size).max())
+        print("n", n, "k", k, "m", m, "worst", worst, flush=True)
+        assert worst <= (k / 16 + 24) * 2.0**-24
+    lin.close()
+
+
+# grids without a K split use no scratch: the first call may be recorded into a graph, and two
+# streams may run one handle at once
+def test_q4_0_rows_capture_and_streams():
+    n, k, m = 16384, 512, 12
+    lin, _ = _raw(hip.FMT_Q4_0, n, k, 2)
+    xs = [torch.randn(m, k, device="cuda", generator=torch.Generator("cuda").manual_seed(i))
+          for i in range(2)]
+    ys = [torch.zeros(m, n, device="cuda") for _ in range(2)]
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=streams[0]):
+        lin.forward_dev(m, xs[0].data_ptr(), ys[0].data_ptr(), stream=streams[0].cuda_stream)
+    want = [torch.from_numpy(lin.forward(x.cpu().numpy())).cuda() for x in xs]
+    for _ in range(3):
+        ys[0].zero_()
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(ys[0], want[0])
+    for _ in range(20):
+        for x, y, s in zip(xs, ys, streams):
+            lin.forward_dev(m, x.data_ptr(), y.data_ptr(), stream=s.cuda_stream)
+    torch.cuda.synchronize()
+    for y, v in zip(ys, want):
+        assert torch.equal(y, v)
     lin.close()
