@@ -128,6 +128,7 @@ __device__ __forceinline__ float kqf_unfix(long long a) {
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef long long i64x2 __attribute__((ext_vector_type(2)));
 
 // 4 x 4 transpose between the four groups of 16 lanes and the elements of v:
 // element g of group s goes to element s of group g

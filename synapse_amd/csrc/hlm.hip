@@ -481,7 +481,7 @@ struct syn_hip_hlm_s {
     SYN_HIP(hipStreamSynchronize(stream));
     rs.cap = 0;
     SYN_TRY(rs.ids.alloc(n * 4));
-    SYN_TRY(rs.x.alloc(n * H * 4));
+    SYN_TRY(rs.x.alloc(n * H * sizeof(long long)));
     SYN_TRY(rs.xf.alloc(rows_frag_bytes(n, kmax, true)));
     SYN_TRY(rs.qrot.alloc(n * qd * 4));
     SYN_TRY(rs.attn.alloc(n * qd * 4));
@@ -504,7 +504,7 @@ struct syn_hip_hlm_s {
     SYN_TRY(set_state((int)n - 1, ids[n - 1], step));
     SYN_HIP(hipMemcpyAsync(rs.ids.p, ids, n * 4, hipMemcpyHostToDevice, stream));
     const int T = (int)n;
-    float *x = rs.x.as<float>();
+    long long *x = rs.x.as<long long>();
     HRows add;  // the last projection's rows, still to be added to x
     for (size_t l = 0; l < L; l++) {
       Layer &Ly = layers[l];

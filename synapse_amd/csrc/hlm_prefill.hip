@@ -24,6 +24,19 @@ __device__ __forceinline__ void hrow_get(const HRows &h, int t, int off, int c, 
   }
 }
 
+// the same columns of each K split added to the residual row r, in the step's
+// fixed point
+__device__ __forceinline__ void hrow_add(const HRows &h, int t, int c, long long (&r)[8]) {
+  const float *p = h.p + (size_t)t * h.ld + 8 * c;
+  for (int z = 0; z < h.kz; z++, p += h.zs) {
+    const float4 a = *reinterpret_cast<const float4 *>(p);
+    const float4 b = *reinterpret_cast<const float4 *>(p + 4);
+    const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+    for (int i = 0; i < 8; i++) r[i] += kqf_fix(v[i]);
+  }
+}
+
 template <int NT>
 __device__ __forceinline__ float block_max(float v, float *red) {
   for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));
@@ -58,7 +71,7 @@ constexpr int kGluNT = 512, kGluR = kHrowsMaxF / 8 / kGluNT;
 
 // one workgroup per row; row values in registers between the reductions
 __global__ void __launch_bounds__(kNormNT)
-    k_hrows_norm(float *__restrict__ x, const float *__restrict__ embed,
+    k_hrows_norm(long long *__restrict__ x, const float *__restrict__ embed,
                  const uint32_t *__restrict__ ids, int vocab, HRows add,
                  const float *__restrict__ gain, float eps, int T, int H, f16x8 *__restrict__ xf,
                  float *__restrict__ rowmul) {
@@ -71,32 +84,38 @@ __global__ void __launch_bounds__(kNormNT)
   for (int j = 0; j < kNormR; j++) {
     const int c = tid + kNormNT * j;
     if (c >= chunks || !real) break;
-    float *xr = x + (size_t)m * H + 8 * c;
-    const float *src = xr;
-    bool in = true;
-    if (ids) {
+    i64x2 *xr = reinterpret_cast<i64x2 *>(x + (size_t)m * H + 8 * c);
+    long long r[8];
+    if (ids) {  // an id outside the vocabulary is a zero row
       const uint32_t id = ids[m];
-      in = id < (uint32_t)vocab;
-      src = embed + (in ? (size_t)id * H : 0) + 8 * c;
+      const bool in = id < (uint32_t)vocab;
+      const float *src = embed + (in ? (size_t)id * H : 0) + 8 * c;
+      const float4 a = *reinterpret_cast<const float4 *>(src);
+      const float4 b = *reinterpret_cast<const float4 *>(src + 4);
+      const float f[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+      for (int i = 0; i < 8; i++) r[i] = in ? kqf_fix(f[i]) : 0;
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const i64x2 q = xr[i];
+        r[2 * i] = q.x;
+        r[2 * i + 1] = q.y;
+      }
     }
-    const float4 a = *reinterpret_cast<const float4 *>(src);
-    const float4 b = *reinterpret_cast<const float4 *>(src + 4);
-    const float f[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-    float d[8] = {};
-    if (add.p) hrow_get(add, m, 0, c, d);
+    if (add.p) hrow_add(add, m, c, r);
     const float4 ga = *reinterpret_cast<const float4 *>(gain + 8 * c);
     const float4 gb = *reinterpret_cast<const float4 *>(gain + 8 * c + 4);
     const float g[8] = {ga.x, ga.y, ga.z, ga.w, gb.x, gb.y, gb.z, gb.w};
 #pragma unroll
     for (int i = 0; i < 8; i++) {
-      const float s = (in ? f[i] : 0.0f) + d[i];
+      const float s = kqf_unfix(r[i]);
       ss += s * s;
-      d[i] = s;
       v[j][i] = s * g[i];
       mx = fmaxf(mx, fabsf(v[j][i]));
     }
-    *reinterpret_cast<float4 *>(xr) = float4{d[0], d[1], d[2], d[3]};
-    *reinterpret_cast<float4 *>(xr + 4) = float4{d[4], d[5], d[6], d[7]};
+#pragma unroll
+    for (int i = 0; i < 4; i++) xr[i] = i64x2{r[2 * i], r[2 * i + 1]};
   }
   for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
   if ((tid & 63) == 0) rss[tid >> 6] = ss;
@@ -188,18 +207,21 @@ __global__ void __launch_bounds__(kGluNT)
 }
 
 __global__ void __launch_bounds__(256)
-    k_hrows_last(const float *__restrict__ x, HRows add, int T, int H, long long *__restrict__ r) {
+    k_hrows_last(const long long *__restrict__ x, HRows add, int T, int H,
+                 long long *__restrict__ r) {
   const int c = blockIdx.x * 256 + threadIdx.x;
   if (8 * c >= H) return;
-  float d[8];
-  hrow_get(add, T - 1, 0, c, d);
+  long long v[8];
 #pragma unroll
-  for (int i = 0; i < 8; i++) r[8 * c + i] = kqf_fix(x[(size_t)(T - 1) * H + 8 * c + i] + d[i]);
+  for (int i = 0; i < 8; i++) v[i] = x[(size_t)(T - 1) * H + 8 * c + i];
+  hrow_add(add, T - 1, c, v);
+#pragma unroll
+  for (int i = 0; i < 8; i++) r[8 * c + i] = v[i];
 }
 
 }  // namespace
 
-syn_status_t launch_hrows_norm(float *x, const float *embed, const uint32_t *ids, int vocab,
+syn_status_t launch_hrows_norm(long long *x, const float *embed, const uint32_t *ids, int vocab,
                                HRows add, const float *gain, float eps, int T, int H, void *xf,
                                hipStream_t s) {
   if (H % 8 || H > kHrowsMaxH) return SYN_ERR_INVALID_ARG;
@@ -228,7 +250,7 @@ syn_status_t launch_hrows_swiglu(HRows gu, int T, int F, void *xf, hipStream_t s
   return SYN_OK;
 }
 
-syn_status_t launch_hrows_last(const float *x, HRows add, int T, int H, long long *r,
+syn_status_t launch_hrows_last(const long long *x, HRows add, int T, int H, long long *r,
                                hipStream_t s) {
   if (H % 8) return SYN_ERR_INVALID_ARG;
   hipLaunchKernelGGL(k_hrows_last, dim3((unsigned)cdiv((size_t)H / 8, 256)), dim3(256), 0, s, x,

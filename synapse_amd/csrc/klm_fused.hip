@@ -128,7 +128,6 @@ __device__ __forceinline__ float wave_max(float v) {
   return fmaxf(fmaxf(lane_f(v, 0), lane_f(v, 16)), fmaxf(lane_f(v, 32), lane_f(v, 48)));
 }
 
-typedef long long i64x2 __attribute__((ext_vector_type(2)));
 
 // 32 activations of a stage from LDS (all lanes read the same address)
 __device__ __forceinline__ void lds_x32(float (&x)[32], const float *src) {
