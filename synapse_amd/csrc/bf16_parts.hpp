@@ -57,4 +57,17 @@ __device__ __forceinline__ bf16x8 q4_levels(uint32_t v) {
   return __builtin_bit_cast(bf16x8, u32x4{o[0], o[1], o[2], o[3]});
 }
 
+// the parts of chunk c (elements 8c .. 8c+7) of row m to their lane's place in
+// the fragments of k_rows_gemm_parts, whose rows have B blocks
+__device__ __forceinline__ void parts_put(bf16x8 *__restrict__ xf, int B, int m, int c,
+                                          const float (&v)[8]) {
+  bf16x8 p[3];
+  bf16_parts(v, p);
+  // block c / 4, half (c / 2) % 2, MFMA c % 2
+  const size_t at = (((size_t)(m >> 5) * B + (c >> 2)) * 2 + (c & 1)) * 3;
+  const int lane = ((c >> 1) & 1) * 32 + (m & 31);
+#pragma unroll
+  for (int i = 0; i < 3; i++) xf[(at + i) * 64 + lane] = p[i];
+}
+
 }  // namespace syn

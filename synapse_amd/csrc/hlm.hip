@@ -244,7 +244,6 @@ struct syn_hip_hlm_s {
   // residual r [H], the split-K accumulator of in_proj / q|k|v (cleared by
   // the projection after its reader), attention chunk partials, lm_head top-2
   bool use_fused = true, fused_ok = false;
-  bool split_ok = true;  // every projection takes the split-f16 product (QLinearQ4_0::split_ok)
   KqfPlan fp_in, fp_out, fp_qkv, fp_o, fp_gu, fp_down;
   DevBuf f_r, f_acc, f_ao, f_aml, f_pv, f_pi, f_pv2;
   size_t n_qkv = 0;
@@ -260,17 +259,14 @@ struct syn_hip_hlm_s {
   // the fused step's plans and buffers, when every shape fits its kernels
   syn_status_t setup_fused() {
     fused_ok = false;
-    split_ok = true;
     const int fm[1] = {SYN_HIP_FMT_Q4_0};
     if (!kqf_fits((int)H, (int)qd, (int)F, (int)nh, (int)nkv, (int)hd, (int)S, fm, 1) ||
         I % 256 || !head_f32_fits((int)H))
       return SYN_OK;
     bool any_conv = false, any_gqa = false;
     for (auto &Ly : layers) {
-      for (QLinearQ4_0 *q : {&Ly.in, &Ly.out, &Ly.qkv, &Ly.o, &Ly.gu, &Ly.down}) {
+      for (QLinearQ4_0 *q : {&Ly.in, &Ly.out, &Ly.qkv, &Ly.o, &Ly.gu, &Ly.down})
         if (q->n && !q->gemm_ok()) return SYN_OK;  // halved subnormal scales
-        if (q->n && !q->split_ok()) split_ok = false;
-      }
       (Ly.kind == 0 ? any_conv : any_gqa) = true;
     }
     const Layer *conv = nullptr, *gqa = nullptr;
@@ -436,8 +432,8 @@ struct syn_hip_hlm_s {
   static constexpr size_t kRowsMax = 2048;
   // Below this many tokens the replayed step is the faster form: a layer of
   // the rows form takes ~65 us at 3-32 tokens, the step ~20 us a token.  LFM2.5
-  // widths, four layers, whole calls: 3 tokens 337 us against 495, 64 tokens
-  // 417 against 9400
+  // widths, four layers, whole calls: 3 tokens 311 us against 495, 64 tokens
+  // 394 against 9400
   static constexpr size_t kRowsMin = 3;
   struct RowsScratch {
     size_t cap = 0;
@@ -449,7 +445,7 @@ struct syn_hip_hlm_s {
   // row kernels' registers and the prompt attention's LDS
   bool rows_supported() const {
     return use_fused && fused_ok && H <= (size_t)kHrowsMaxH && I <= (size_t)kHrowsMaxH &&
-           qd <= (size_t)kHrowsMaxH && F <= (size_t)kHrowsMaxF && split_ok;
+           qd <= (size_t)kHrowsMaxH && F <= (size_t)kHrowsMaxF;
   }
   static RowsGemm rows_of(const QLinearQ4_0 &q) {
     RowsGemm g;
@@ -468,7 +464,7 @@ struct syn_hip_hlm_s {
       for (QLinearQ4_0 *q : {&Ly.in, &Ly.out, &Ly.qkv, &Ly.o, &Ly.gu, &Ly.down}) {
         if (!q->n) continue;
         kmax = std::max(kmax, q->k);
-        part = std::max(part, n * q->n * (size_t)rows_gemm_splits(rows_of(*q), n, true));
+        part = std::max(part, n * q->n * (size_t)rows_parts_splits(rows_of(*q), n));
       }
     if (rs.part_elems < part) {
       SYN_HIP(hipStreamSynchronize(stream));
@@ -482,19 +478,19 @@ struct syn_hip_hlm_s {
     rs.cap = 0;
     SYN_TRY(rs.ids.alloc(n * 4));
     SYN_TRY(rs.x.alloc(n * H * sizeof(long long)));
-    SYN_TRY(rs.xf.alloc(rows_frag_bytes(n, kmax, true)));
+    SYN_TRY(rs.xf.alloc(rows_parts_bytes(n, kmax)));
     SYN_TRY(rs.qrot.alloc(n * qd * 4));
     SYN_TRY(rs.attn.alloc(n * qd * 4));
     rs.cap = n;
     return SYN_OK;
   }
 
-  // rs.part = the fragments in rs.xf times W^T, in at most kz K splits
+  // rs.part = the rows in rs.xf times W^T, in at most kz K splits
   syn_status_t rows_gemm(const QLinearQ4_0 &q, size_t n, int kz, HRows *out) {
     const RowsGemm g = rows_of(q);
-    kz = std::min(kz, rows_gemm_splits(g, n, true));
+    kz = std::min(kz, rows_parts_splits(g, n));
     *out = HRows{rs.part.as<float>(), kz, n * q.n, (int)q.n};
-    return launch_rows_gemm_split(g, rs.xf.p, n, kz, rs.part.as<float>(), q.n, n * q.n, stream);
+    return launch_rows_gemm_parts(g, rs.xf.p, n, kz, rs.part.as<float>(), q.n, n * q.n, stream);
   }
 
   // every layer over ids[0..n) at positions 0.., then the lm_head and argmax
@@ -529,8 +525,7 @@ struct syn_hip_hlm_s {
         SYN_TRY(launch_attention_prefill_tol(rs.qrot.as<float>(), Ly.kc.as<float>(),
                                              Ly.vc.as<float>(), T, (int)nh, (int)nkv, (int)hd,
                                              (int)S, rs.attn.as<float>(), stream));
-        SYN_TRY(launch_rows_frag(SYN_HIP_FMT_Q4_0, rs.attn.as<float>(), qd, n, qd, true, rs.xf.p,
-                                 nullptr, 0, 0, stream));
+        SYN_TRY(launch_rows_parts(rs.attn.as<float>(), qd, n, qd, rs.xf.p, stream));
         SYN_TRY(rows_gemm(Ly.o, n, kRowsMaxSplit, &add));
       }
       SYN_TRY(launch_hrows_norm(x, nullptr, nullptr, 0, add, Ly.ffn_nw.as<float>(), c.eps, T,

@@ -1,11 +1,11 @@
 // The hybrid (LFM2.5) layers over the rows of a prompt.  Token by token a
 // prompt reads every weight and the 268 MB lm_head once per token (~0.15 ms at
-// four layers); here the projections are split-f16 matrix products over all
-// tokens (rows_gemm.hip: as accurate as the step's f32 sums), and the ops
-// between them are one kernel each that sums the product's K splits, computes
-// its rows and writes the next product's activation fragments directly.
+// four layers); here the projections are matrix products over all tokens that
+// round nothing before their f32 sums (rows_gemm.hip), and the ops between them
+// are one kernel each that sums the product's K splits, computes its rows and
+// writes the next product's activation parts directly.
+#include "bf16_parts.hpp"
 #include "hlm_prefill.hpp"
-#include "rows_frag.hpp"
 
 namespace syn {
 
@@ -37,32 +37,18 @@ __device__ __forceinline__ void hrow_add(const HRows &h, int t, int c, long long
   }
 }
 
-template <int NT>
-__device__ __forceinline__ float block_max(float v, float *red) {
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < NT / 64; i++) v = fmaxf(v, red[i]);
-  return v;
-}
-
-// scale the thread's chunks tid, tid + NT, .. by the row's power of two and
-// write them (zeros for the padding rows of the last tile)
+// the parts of the thread's chunks tid, tid + NT, .. (zeros for the padding
+// rows of the last tile)
 template <int NT, int R>
-__device__ __forceinline__ void put_row(float (&v)[R][8], int chunks, float mx, bool real, int m,
-                                        f16x8 *__restrict__ xf, float *__restrict__ rowmul) {
-  float up, down;
-  frag_row_scale(mx, &up, &down);
-  if (threadIdx.x == 0) rowmul[m] = down;
-  const int steps = (8 * chunks + kFragStep - 1) / kFragStep;
+__device__ __forceinline__ void put_row(const float (&v)[R][8], int chunks, bool real, int m,
+                                        bf16x8 *__restrict__ xf) {
+  const float zero[8] = {};
 #pragma unroll
   for (int j = 0; j < R; j++) {
     const int c = threadIdx.x + NT * j;
     if (c >= chunks) break;
-#pragma unroll
-    for (int i = 0; i < 8; i++) v[j][i] = real ? v[j][i] * up : 0.0f;
-    frag_put<true, true>(xf, steps, m, c, v[j]);
+    if (real) parts_put(xf, chunks >> 2, m, c, v[j]);
+    else parts_put(xf, chunks >> 2, m, c, zero);
   }
 }
 
@@ -73,13 +59,12 @@ constexpr int kGluNT = 512, kGluR = kHrowsMaxF / 8 / kGluNT;
 __global__ void __launch_bounds__(kNormNT)
     k_hrows_norm(long long *__restrict__ x, const float *__restrict__ embed,
                  const uint32_t *__restrict__ ids, int vocab, HRows add,
-                 const float *__restrict__ gain, float eps, int T, int H, f16x8 *__restrict__ xf,
-                 float *__restrict__ rowmul) {
-  __shared__ float red[kNormNT / 64], rss[kNormNT / 64];
+                 const float *__restrict__ gain, float eps, int T, int H, bf16x8 *__restrict__ xf) {
+  __shared__ float rss[kNormNT / 64];
   const int m = blockIdx.x, tid = threadIdx.x, chunks = H >> 3;
   const bool real = m < T;
   float v[kNormR][8];
-  float ss = 0.0f, mx = 0.0f;
+  float ss = 0.0f;
 #pragma unroll
   for (int j = 0; j < kNormR; j++) {
     const int c = tid + kNormNT * j;
@@ -112,14 +97,13 @@ __global__ void __launch_bounds__(kNormNT)
       const float s = kqf_unfix(r[i]);
       ss += s * s;
       v[j][i] = s * g[i];
-      mx = fmaxf(mx, fabsf(v[j][i]));
     }
 #pragma unroll
     for (int i = 0; i < 4; i++) xr[i] = i64x2{r[2 * i], r[2 * i + 1]};
   }
   for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
   if ((tid & 63) == 0) rss[tid >> 6] = ss;
-  mx = block_max<kNormNT>(mx, red);
+  __syncthreads();
   ss = 0.0f;
 #pragma unroll
   for (int i = 0; i < kNormNT / 64; i++) ss += rss[i];
@@ -128,7 +112,7 @@ __global__ void __launch_bounds__(kNormNT)
   for (int j = 0; j < kNormR; j++)
 #pragma unroll
     for (int i = 0; i < 8; i++) v[j][i] *= scale;
-  put_row<kNormNT>(v, chunks, mx * scale, real, m, xf, rowmul);
+  put_row<kNormNT>(v, chunks, real, m, xf);
 }
 
 // layer.rs:25-42, 609-627 over the prompt: taps oldest to newest, zeros before
@@ -136,13 +120,10 @@ __global__ void __launch_bounds__(kNormNT)
 // products a channel) rather than in a pass of their own
 __global__ void __launch_bounds__(kNormNT)
     k_hrows_conv(HRows p, const float *__restrict__ w, const float *__restrict__ bias, int T,
-                 int I, int ck, float *__restrict__ state, f16x8 *__restrict__ xf,
-                 float *__restrict__ rowmul) {
-  __shared__ float red[kNormNT / 64];
+                 int I, int ck, float *__restrict__ state, bf16x8 *__restrict__ xf) {
   const int m = blockIdx.x, tid = threadIdx.x, chunks = I >> 3;
   const bool real = m < T;
   float v[kNormR][8];
-  float mx = 0.0f;
 #pragma unroll
   for (int j = 0; j < kNormR; j++) {
     const int c = tid + kNormNT * j;
@@ -170,25 +151,20 @@ __global__ void __launch_bounds__(kNormNT)
     float gate[8];
     hrow_get(p, m, I, c, gate);
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
+    for (int i = 0; i < 8; i++)
       v[j][i] = gate[i] * (bias ? sum[i] + bias[8 * c + i] : sum[i]);
-      mx = fmaxf(mx, fabsf(v[j][i]));
-    }
   }
-  mx = block_max<kNormNT>(mx, red);
-  put_row<kNormNT>(v, chunks, mx, real, m, xf, rowmul);
+  put_row<kNormNT>(v, chunks, real, m, xf);
 }
 
 __global__ void __launch_bounds__(kGluNT)
-    k_hrows_swiglu(HRows gu, int T, int F, f16x8 *__restrict__ xf, float *__restrict__ rowmul) {
-  __shared__ float red[kGluNT / 64];
+    k_hrows_swiglu(HRows gu, int T, int F, bf16x8 *__restrict__ xf) {
   __shared__ uint64_t etab[32];
   const int m = blockIdx.x, tid = threadIdx.x, chunks = F >> 3;
   const bool real = m < T;
   if (tid < 32) etab[tid] = syn_exp2_tab[tid];
   __syncthreads();
   float v[kGluR][8];
-  float mx = 0.0f;
 #pragma unroll
   for (int j = 0; j < kGluR; j++) {
     const int c = tid + kGluNT * j;
@@ -197,13 +173,9 @@ __global__ void __launch_bounds__(kGluNT)
     hrow_get(gu, m, 0, c, g);
     hrow_get(gu, m, F, c, u);
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-      v[j][i] = syn_silu_tab(g[i], etab) * u[i];
-      mx = fmaxf(mx, fabsf(v[j][i]));
-    }
+    for (int i = 0; i < 8; i++) v[j][i] = syn_silu_tab(g[i], etab) * u[i];
   }
-  mx = block_max<kGluNT>(mx, red);
-  put_row<kGluNT>(v, chunks, mx, real, m, xf, rowmul);
+  put_row<kGluNT>(v, chunks, real, m, xf);
 }
 
 __global__ void __launch_bounds__(256)
@@ -224,28 +196,26 @@ __global__ void __launch_bounds__(256)
 syn_status_t launch_hrows_norm(long long *x, const float *embed, const uint32_t *ids, int vocab,
                                HRows add, const float *gain, float eps, int T, int H, void *xf,
                                hipStream_t s) {
-  if (H % 8 || H > kHrowsMaxH) return SYN_ERR_INVALID_ARG;
+  if (H % 32 || H > kHrowsMaxH) return SYN_ERR_INVALID_ARG;
   hipLaunchKernelGGL(k_hrows_norm, dim3((unsigned)round_up(T, 32)), dim3(kNormNT), 0, s, x, embed,
-                     ids, vocab, add, gain, eps, T, H, static_cast<f16x8 *>(xf),
-                     rows_frag_scales(xf, T, H, true));
+                     ids, vocab, add, gain, eps, T, H, static_cast<bf16x8 *>(xf));
   SYN_LAUNCH_CHECK();
   return SYN_OK;
 }
 
 syn_status_t launch_hrows_conv(HRows p, const float *w, const float *bias, int T, int I, int ck,
                                float *state, void *xf, hipStream_t s) {
-  if (I % 8 || I > kHrowsMaxH) return SYN_ERR_INVALID_ARG;
+  if (I % 32 || I > kHrowsMaxH) return SYN_ERR_INVALID_ARG;
   hipLaunchKernelGGL(k_hrows_conv, dim3((unsigned)round_up(T, 32)), dim3(kNormNT), 0, s, p, w,
-                     bias, T, I, ck, state, static_cast<f16x8 *>(xf),
-                     rows_frag_scales(xf, T, I, true));
+                     bias, T, I, ck, state, static_cast<bf16x8 *>(xf));
   SYN_LAUNCH_CHECK();
   return SYN_OK;
 }
 
 syn_status_t launch_hrows_swiglu(HRows gu, int T, int F, void *xf, hipStream_t s) {
-  if (F % 8 || F > kHrowsMaxF) return SYN_ERR_INVALID_ARG;
+  if (F % 32 || F > kHrowsMaxF) return SYN_ERR_INVALID_ARG;
   hipLaunchKernelGGL(k_hrows_swiglu, dim3((unsigned)round_up(T, 32)), dim3(kGluNT), 0, s, gu, T, F,
-                     static_cast<f16x8 *>(xf), rows_frag_scales(xf, T, F, true));
+                     static_cast<bf16x8 *>(xf));
   SYN_LAUNCH_CHECK();
   return SYN_OK;
 }

@@ -880,7 +880,7 @@ __global__ void __launch_bounds__(256)
 // power of two whose inverse lands in *rowmul (m floats after the rows), in
 // the k_gemm_kqr Q4_0 chunk order if perm8
 size_t f16_rows_bytes(size_t m, size_t k) {
-  // also rows_frag_bytes(m, k, false), whose rows are whole 32-row tiles
+  // also rows_frag_bytes(m, k), whose rows are whole 32-row tiles
   return round_up(round_up(m, 32) * round_up(k, PGK) * 2, 256) + round_up(m, 32) * sizeof(float);
 }
 static syn_status_t ensure_rows(size_t need, DevBuf &xh, size_t &xh_bytes) {
@@ -958,9 +958,9 @@ static syn_status_t kq_gemm_f16(int fmt, bool exact, const u32x4 *W, const uint1
     const bool can_split =
         ldy % 4 == 0 && reinterpret_cast<uintptr_t>(d_y) % 16 == 0 &&
         !rows_overlap(d_x, m, k, ldx, d_y, n, ldy);
-    const int kz = can_split ? rows_gemm_splits(g, m, false) : 1;
+    const int kz = can_split ? rows_gemm_splits(g, m) : 1;
     SYN_TRY(ensure_rows(f16_rows_bytes(m, k), xh, xh_bytes));
-    SYN_TRY(launch_rows_frag(fmt, d_x, ldx, m, k, false, xh.p, kz > 1 ? d_y : nullptr, ldy, n, s));
+    SYN_TRY(launch_rows_frag(fmt, d_x, ldx, m, k, xh.p, kz > 1 ? d_y : nullptr, ldy, n, s));
     return launch_rows_gemm(g, xh.p, m, kz, d_y, ldy, s);
   }
   // dynamic-LDS attribute set per kernel: k_gemm_kq5 0-3 and 8, k_gemm_kqr

@@ -126,7 +126,6 @@ struct QLinearQ4_0 {
   // reference's GGUF Q4_0 path; false = the Zig GEMV's IEEE conversion
   bool rs_f16_scales = false;
   bool has_subnormal_scale = false;  // some block scale is an f16 subnormal (set at upload)
-  bool has_wide_scale = false;  // 8 d is beyond f16 for some block scale d, or d is not finite
   DevBuf xh;                         // f16 activations for the MFMA GEMM
   size_t xh_bytes = 0;  // its size (f16_rows_bytes)
   SplitKSlots sk;  // gemv()'s one-launch K split (split_k.hpp)
@@ -153,8 +152,6 @@ struct QLinearQ4_0 {
   syn_status_t ensure_slots();
   // the GEMM decodes the scales as IEEE f16 values: not for halved subnormals
   bool gemm_ok() const { return !(rs_f16_scales && has_subnormal_scale); }
-  // the split form also needs (nibble - 8) * d within f16's range
-  bool split_ok() const { return gemm_ok() && !has_wide_scale; }
 };
 
 // Ternary linear: TernaryLinear (ternary_linear.rs); f32 activations.

@@ -19,8 +19,8 @@
 // then its high ones).
 #include <algorithm>
 
+#include "bf16_parts.hpp"
 #include "kquant.hpp"
-#include "rows_frag.hpp"
 #include "rows_gemm.hpp"
 
 namespace syn {
@@ -28,11 +28,12 @@ namespace syn {
 namespace {
 
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int RW = 8;        // waves per workgroup
 constexpr int RNT = 64 * RW;
-constexpr int KSTEP = kFragStep;
+constexpr int KSTEP = 64;  // elements of K per step
 
 constexpr bool nibble_order(int fmt) { return fmt != SYN_HIP_FMT_Q8_0; }
 
@@ -135,11 +136,9 @@ __device__ __forceinline__ Scale scale_of(const Raw<FMT> &r, int B, int step, in
 }
 
 // the lane's eight weights of group g, each the dequantizer's value rounded
-// once to f16; lo (Q4_0): what that rounding left, exact (a product of 4 and
-// 11 significant bits is the sum of two f16)
-template <int FMT, bool SPLIT>
-__device__ __forceinline__ void decode(const Raw<FMT> &r, const Scale &s, int g, f16x8 &hi,
-                                       f16x8 &lo) {
+// once to f16
+template <int FMT>
+__device__ __forceinline__ f16x8 decode(const Raw<FMT> &r, const Scale &s, int g) {
   uint32_t o[4];
   if constexpr (FMT == SYN_HIP_FMT_Q4_0) {
     const f16x2 bias = f16x2{(_Float16)-1032.0f, (_Float16)-1032.0f};
@@ -149,16 +148,9 @@ __device__ __forceinline__ void decode(const Raw<FMT> &r, const Scale &s, int g,
                            __builtin_amdgcn_perm(0x64646464u, l, 0x04030402u),
                            __builtin_amdgcn_perm(0x64646464u, h, 0x04010400u),
                            __builtin_amdgcn_perm(0x64646464u, h, 0x04030402u)};
-    uint32_t e[4];
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const f16x2 q = __builtin_bit_cast(f16x2, p[i]) + bias;
-      const f16x2 w = q * s.d;
-      o[i] = __builtin_bit_cast(uint32_t, w);
-      if constexpr (SPLIT)
-        e[i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(q, s.d, -w));
-    }
-    if constexpr (SPLIT) lo = __builtin_bit_cast(f16x8, u32x4{e[0], e[1], e[2], e[3]});
+    for (int i = 0; i < 4; i++)
+      o[i] = __builtin_bit_cast(uint32_t, (__builtin_bit_cast(f16x2, p[i]) + bias) * s.d);
   } else if constexpr (FMT == SYN_HIP_FMT_Q8_0) {
     const f16x2 bias = f16x2{(_Float16)-1152.0f, (_Float16)-1152.0f};
 #pragma unroll
@@ -194,21 +186,56 @@ __device__ __forceinline__ void decode(const Raw<FMT> &r, const Scale &s, int g,
       o[2 + i] = pk(val(h, 2 * i), val(h, 2 * i + 1));
     }
   }
-  hi = __builtin_bit_cast(f16x8, u32x4{o[0], o[1], o[2], o[3]});
+  return __builtin_bit_cast(f16x8, u32x4{o[0], o[1], o[2], o[3]});
 }
 
-// grid (ceil(N / 32 NT), ceil(M / 32 MT), K splits)
-// SPLIT: activations and weights as sums of two f16, three products (the
-// fourth, of the two remainders, is below an f32 rounding).  zs: elements
-// between the K splits' outputs in y, or 0 to add them into one
-template <int FMT, int MT, int NT, bool SPLIT>
+// the eight waves' sums: the upper four through LDS into the lower four, then
+// store(row, column, sum) of the tile's elements, one thread each
+template <int MT, int NT, class Store>
+__device__ __forceinline__ void sum_waves(f32x16 (&acc)[MT][NT],
+                                          float (&red)[RW / 2][32 * MT][32 * NT + 8],
+                                          Store store) {
+  const int tid = threadIdx.x, l32 = tid & 31, lh = (tid >> 5) & 1;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  auto at = [&](int slot, int mt, int nt, int r) -> float & {
+    return red[slot][32 * mt + 8 * (r >> 2) + 4 * lh + (r & 3)][32 * nt + l32];
+  };
+  auto put = [&](int slot) {
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+      for (int nt = 0; nt < NT; nt++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) at(slot, mt, nt, r) = acc[mt][nt][r];
+  };
+  if (wave >= RW / 2) put(wave - RW / 2);
+  __syncthreads();
+  if (wave < RW / 2) {
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+      for (int nt = 0; nt < NT; nt++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[mt][nt][r] += at(wave, mt, nt, r);
+    put(wave);
+  }
+  __syncthreads();
+  for (int i = tid; i < 32 * MT * 32 * NT; i += RNT) {
+    const int r = i / (32 * NT), c = i % (32 * NT);
+    float t = red[0][r][c];
+#pragma unroll
+    for (int w = 1; w < RW / 2; w++) t += red[w][r][c];
+    store(r, c, t);
+  }
+}
+
+// grid (ceil(N / 32 NT), ceil(M / 32 MT), K splits, added into y)
+template <int FMT, int MT, int NT>
 __global__ void __launch_bounds__(RNT) __attribute__((amdgpu_waves_per_eu(2, 2)))
     k_rows_gemm(const u32x4 *__restrict__ W, const uint16_t *__restrict__ Wd, int N, int B,
                 const f16x8 *__restrict__ xf, const float *__restrict__ rowmul, int M, int steps,
-                int per, float *__restrict__ y, int ldy, size_t zs) {
-  constexpr int AP = SPLIT ? 2 : 1;
-  constexpr int CP = 32 * NT + 8;  // column pitch of the reduction rows
-  __shared__ float red[RW / 2][32 * MT][CP];
+                int per, float *__restrict__ y, int ldy) {
+  __shared__ float red[RW / 2][32 * MT][32 * NT + 8];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, lh = lane >> 5;
@@ -228,7 +255,7 @@ __global__ void __launch_bounds__(RNT) __attribute__((amdgpu_waves_per_eu(2, 2))
   const f16x8 *xt[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; mt++)
-    xt[mt] = xf + (size_t)min(mt0 + mt, mlast) * steps * (256 * AP) + lane;
+    xt[mt] = xf + (size_t)min(mt0 + mt, mlast) * steps * 256 + lane;
   f32x16 acc[MT][NT];
 #pragma unroll
   for (int mt = 0; mt < MT; mt++)
@@ -238,7 +265,7 @@ __global__ void __launch_bounds__(RNT) __attribute__((amdgpu_waves_per_eu(2, 2))
       for (int r = 0; r < 16; r++) acc[mt][nt][r] = 0.0f;
   struct Step {
     Raw<FMT> w[NT];
-    f16x8 a[MT][4][AP];
+    f16x8 a[MT][4];
   };
   auto load = [&](Step &st, int step) {
 #pragma unroll
@@ -247,10 +274,7 @@ __global__ void __launch_bounds__(RNT) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
     for (int mt = 0; mt < MT; mt++)
 #pragma unroll
-      for (int g = 0; g < 4; g++)
-#pragma unroll
-        for (int p = 0; p < AP; p++)
-          st.a[mt][g][p] = xt[mt][(size_t)step * (256 * AP) + (g * AP + p) * 64];
+      for (int g = 0; g < 4; g++) st.a[mt][g] = xt[mt][(size_t)step * 256 + g * 64];
   };
   auto mul = [&](const Step &st, int step) {
 #pragma unroll
@@ -258,25 +282,18 @@ __global__ void __launch_bounds__(RNT) __attribute__((amdgpu_waves_per_eu(2, 2))
       const Scale sc = scale_of<FMT>(st.w[nt], B, step, lh);
 #pragma unroll
       for (int g = 0; g < 4; g++) {
-        f16x8 b, b2;
-        decode<FMT, SPLIT>(st.w[nt], sc, g, b, b2);
+        const f16x8 b = decode<FMT>(st.w[nt], sc, g);
 #pragma unroll
-        for (int mt = 0; mt < MT; mt++) {
-          f32x16 &c = acc[mt][nt];
-          if constexpr (SPLIT) {
-            c = __builtin_amdgcn_mfma_f32_32x32x16_f16(st.a[mt][g][0], b2, c, 0, 0, 0);
-            c = __builtin_amdgcn_mfma_f32_32x32x16_f16(st.a[mt][g][1], b, c, 0, 0, 0);
-          }
-          c = __builtin_amdgcn_mfma_f32_32x32x16_f16(st.a[mt][g][0], b, c, 0, 0, 0);
-        }
+        for (int mt = 0; mt < MT; mt++)
+          acc[mt][nt] =
+              __builtin_amdgcn_mfma_f32_32x32x16_f16(st.a[mt][g], b, acc[mt][nt], 0, 0, 0);
       }
     }
   };
   // Two steps in flight; the loads past the last step repeat it.  Without
   // the scheduling barriers and the occupancy bound the compiler sinks a
   // step's loads to their use to save registers, and every step waits out a
-  // whole load (Q4_0 with split values, 9 rows, 14336 -> 4096: 62 us against
-  // 30).  Three and four steps in flight measured the same or slower.
+  // whole load.  Three and four steps in flight measured the same or slower.
   auto hold = [] { __builtin_amdgcn_sched_barrier(0); };
   Step st0, st1;
   int step = s0 + wave;
@@ -294,44 +311,152 @@ __global__ void __launch_bounds__(RNT) __attribute__((amdgpu_waves_per_eu(2, 2))
       load(st1, min(step + RW, s1 - 1)); hold();
     }
   }
-  // the eight waves' sums: the upper four through LDS into the lower four,
-  // then every thread adds the four
-  auto put = [&](int slot) {
-#pragma unroll
-    for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-      for (int nt = 0; nt < NT; nt++)
-#pragma unroll
-        for (int r = 0; r < 16; r++)
-          red[slot][32 * mt + 8 * (r >> 2) + 4 * lh + (r & 3)][32 * nt + l32] = acc[mt][nt][r];
-  };
-  if (wave >= RW / 2) put(wave - RW / 2);
-  __syncthreads();
-  if (wave < RW / 2) {
-#pragma unroll
-    for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-      for (int nt = 0; nt < NT; nt++)
-#pragma unroll
-        for (int r = 0; r < 16; r++)
-          acc[mt][nt][r] +=
-              red[wave][32 * mt + 8 * (r >> 2) + 4 * lh + (r & 3)][32 * nt + l32];
-    put(wave);
-  }
-  __syncthreads();
-  const bool atomic = gridDim.z > 1 && zs == 0;
-  y += blockIdx.z * zs;
-  for (int i = tid; i < 32 * MT * 32 * NT; i += RNT) {
-    const int r = i / (32 * NT), c = i % (32 * NT);
+  const bool atomic = gridDim.z > 1;
+  sum_waves<MT, NT>(acc, red, [&](int r, int c, float t) {
     const int m = mt0 * 32 + r, n = n0 + c;
-    if (m >= M || n >= N) continue;
-    float t = red[0][r][c];
-#pragma unroll
-    for (int w = 1; w < RW / 2; w++) t += red[w][r][c];
+    if (m >= M || n >= N) return;
     const float v = t * rowmul[m];
     if (atomic) atomicAdd(&y[(size_t)m * ldy + n], v);
     else y[(size_t)m * ldy + n] = v;
+  });
+}
+
+// The same from rows kept whole (bf16_parts.hpp) against Q4_0's levels: a step
+// is one block, its dot six MFMAs, scaled in f32 into the sum.  Lane l < 32
+// holds dwords 0 and 1 of a block's levels, the others 2 and 3, so the
+// activations of MFMA j are elements 8 (2 lh + j) .. +7.  PF steps in flight.
+// Bound by the activations' way from L2, six bytes an element for every tile of
+// columns: 64 rows, the four projections of an LFM2.5 conv layer, 64 columns a
+// workgroup where that is a round of workgroups (a prompt of 64 tokens and four
+// layers 394 us, 512 tokens 908; 412 and 978 with 32 columns, 374 and 840 with
+// operands of two f16, which round the activations to 22 bits).
+// grid (ceil(N / 32 NT), ceil(M / 32 MT), K splits); split z writes y + z zs
+template <int MT, int NT, int PF>
+__global__ void __launch_bounds__(RNT) __attribute__((amdgpu_waves_per_eu(2, 2)))
+    k_rows_gemm_parts(const uint2 *__restrict__ W, const uint16_t *__restrict__ Wd, int N, int B,
+                      const bf16x8 *__restrict__ xf, int M, int per, float *__restrict__ y,
+                      int ldy, size_t zs) {
+  __shared__ float red[RW / 2][32 * MT][32 * NT + 8];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, lh = lane >> 5;
+  const int n0 = blockIdx.x * 32 * NT, mt0 = blockIdx.y * MT;
+  const int s0 = blockIdx.z * per, s1 = min(B, s0 + per);
+  const int last = ((N + 63) >> 6) * 64 - 1, mlast = ((M + 31) >> 5) - 1;
+  size_t at[NT];
+#pragma unroll
+  for (int nt = 0; nt < NT; nt++) {
+    const int n = min(n0 + 32 * nt + l32, last);
+    at[nt] = (size_t)(n >> 6) * B * 64 + (n & 63);
   }
+  const bf16x8 *xt[MT];
+#pragma unroll
+  for (int mt = 0; mt < MT; mt++)
+    xt[mt] = xf + (size_t)min(mt0 + mt, mlast) * B * 384 + lane;
+  f32x16 acc[MT][NT];
+#pragma unroll
+  for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+    for (int nt = 0; nt < NT; nt++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) acc[mt][nt][r] = 0.0f;
+  struct Step {
+    uint2 q[NT];
+    uint16_t d[NT];
+    bf16x8 a[MT][2][3];
+  };
+  auto load = [&](Step &st, int b) {
+#pragma unroll
+    for (int nt = 0; nt < NT; nt++) {
+      st.q[nt] = W[(at[nt] + (size_t)b * 64) * 2 + lh];
+      st.d[nt] = Wd[at[nt] + (size_t)b * 64];
+    }
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+      for (int j = 0; j < 2; j++)
+#pragma unroll
+        for (int i = 0; i < 3; i++) st.a[mt][j][i] = xt[mt][(size_t)b * 384 + (j * 3 + i) * 64];
+  };
+  auto mul = [&](const Step &st) {
+#pragma unroll
+    for (int nt = 0; nt < NT; nt++) {
+      const bf16x8 w[2] = {q4_levels(st.q[nt].x), q4_levels(st.q[nt].y)};
+      const float d = (float)__builtin_bit_cast(_Float16, st.d[nt]);
+      f32x16 dot[MT];
+#pragma unroll
+      for (int mt = 0; mt < MT; mt++) dot[mt] = f32x16{};
+#pragma unroll
+      for (int i = 2; i >= 0; i--)
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+          for (int mt = 0; mt < MT; mt++)
+            dot[mt] =
+                __builtin_amdgcn_mfma_f32_32x32x16_bf16(st.a[mt][j][i], w[j], dot[mt], 0, 0, 0);
+#pragma unroll
+      for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+        for (int r = 0; r < 16; r++)
+          acc[mt][nt][r] = __builtin_fmaf(dot[mt][r], d, acc[mt][nt][r]);
+    }
+  };
+  auto hold = [] { __builtin_amdgcn_sched_barrier(0); };
+  Step st[PF];
+  int b = s0 + wave;
+  if (b < s1) {
+#pragma unroll
+    for (int u = 0; u < PF; u++) {
+      load(st[u], min(b + u * RW, s1 - 1));
+      hold();
+    }
+    for (bool more = true; more;) {
+#pragma unroll
+      for (int u = 0; u < PF; u++) {
+        mul(st[u]);
+        b += RW;
+        if (b >= s1) {
+          more = false;
+          break;
+        }
+        load(st[u], min(b + (PF - 1) * RW, s1 - 1));
+        hold();
+      }
+    }
+  }
+  y += blockIdx.z * zs;
+  sum_waves<MT, NT>(acc, red, [&](int r, int c, float t) {
+    const int m = mt0 * 32 + r, n = n0 + c;
+    if (m < M && n < N) y[(size_t)m * ldy + n] = t * kPartsDown;
+  });
+}
+
+// the power of two that puts mx in [2^14, 2^15) and its inverse; 1 for a row
+// of zeros, at most 2^126.  A row with an infinity (mx; a NaN does not reach
+// it) takes the scale of the largest finite values, so that those stay finite
+__device__ __forceinline__ void frag_row_scale(float mx, float *up, float *down) {
+  *up = *down = 1.0f;
+  if (mx > 0.0f) {
+    int e = 128;
+    if (mx <= 3.4028235e38f) (void)frexpf(mx, &e);
+    e = max(e, 15 - 126);
+    *up = ldexpf(1.0f, 15 - e);
+    *down = ldexpf(1.0f, e - 15);
+  }
+}
+
+// chunk c (elements 8c .. 8c+7, already scaled) of row m to its lane's place.
+// PERM: the nibble formats' k order 0,2,4,6,1,3,5,7
+template <bool PERM>
+__device__ __forceinline__ void frag_put(f16x8 *__restrict__ xf, int steps, int m, int c,
+                                         const float (&v)[8]) {
+  constexpr int ord[8] = {0, 2, 4, 6, 1, 3, 5, 7};
+  f16x8 h;
+#pragma unroll
+  for (int i = 0; i < 8; i++) h[i] = (_Float16)v[PERM ? ord[i] : i];
+  // step c / 8, half (c / 4) % 2, group c % 4
+  const size_t at = ((size_t)(m >> 5) * steps + (c >> 3)) * 4 + (c & 3);
+  xf[at * 64 + ((c >> 2) & 1) * 32 + (m & 31)] = h;
 }
 
 // One workgroup per row (the padding rows of the last tile are zeros): the
@@ -339,7 +464,7 @@ __global__ void __launch_bounds__(RNT) __attribute__((amdgpu_waves_per_eu(2, 2))
 // up to 16384 elements is read once, into registers.
 constexpr int FNT = 512;
 
-template <bool PERM, bool SPLIT>
+template <bool PERM>
 __global__ void __launch_bounds__(FNT)
     k_rows_frag(const float *__restrict__ x, int ldx, int M, int K, int steps,
                 f16x8 *__restrict__ xf, float *__restrict__ rowmul, float *__restrict__ y0,
@@ -392,7 +517,7 @@ __global__ void __launch_bounds__(FNT)
     float t[8];
 #pragma unroll
     for (int i = 0; i < 8; i++) t[i] = m < M ? v[i] * up : 0.0f;
-    frag_put<PERM, SPLIT>(xf, steps, m, c, t);
+    frag_put<PERM>(xf, steps, m, c, t);
   };
 #pragma unroll
   for (int j = 0; j < R; j++)
@@ -407,6 +532,23 @@ __global__ void __launch_bounds__(FNT)
 }
 
 
+// f32 rows -> parts, a thread per chunk of eight values
+__global__ void __launch_bounds__(256)
+    k_rows_parts(const float *__restrict__ x, int ldx, int M, int chunks,
+                 bf16x8 *__restrict__ xf) {
+  const int c = blockIdx.x * 256 + threadIdx.x, m = blockIdx.y;
+  if (c >= chunks) return;
+  float v[8] = {};
+  if (m < M) {
+    const float4 *p = reinterpret_cast<const float4 *>(x + (size_t)m * ldx + 8 * c);
+    const float4 a = p[0], b = p[1];
+    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+    v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+  }
+  parts_put(xf, chunks >> 2, m, c, v);
+}
+
+
 // Columns per workgroup and K splits (at least two steps per wave) with the
 // least time by this count, in steps of a 32-column wave (~0.8 us each): 256
 // CUs take one workgroup at a time, a workgroup costs four steps beside its
@@ -417,14 +559,13 @@ __global__ void __launch_bounds__(FNT)
 struct Shape {
   int mt, nt, kz, per;
 };
-Shape shape_of(const RowsGemm &g, size_t m, int kz_max, bool split) {
+Shape shape_of(const RowsGemm &g, size_t m, int kz_max, bool parts) {
   Shape o{};
   const int steps = (int)cdiv(g.k, KSTEP);
   o.mt = m > 32 ? 2 : 1;
   const int tiles_m = (int)cdiv(m, (size_t)(32 * o.mt));
   float best = 0.0f;
   for (int nt = 1; nt <= 2; nt++) {
-    if (nt == 2 && split && o.mt == 2) break;  // would not fit the registers
     const size_t tiles = cdiv(g.n, (size_t)(32 * nt)) * tiles_m;
     for (int kz = 1; kz <= std::min(kz_max, std::max(1, steps / (2 * RW))); kz++) {
       const float own = (float)cdiv((size_t)steps, (size_t)(RW * kz)) * (nt == 2 ? 1.75f : 1.0f);
@@ -442,43 +583,33 @@ Shape shape_of(const RowsGemm &g, size_t m, int kz_max, bool split) {
   return o;
 }
 
-size_t frag_halfs(size_t m, size_t k, bool split) {
-  return round_up(m, 32) * round_up(k, KSTEP) * (split ? 2 : 1);
+size_t frag_halfs(size_t m, size_t k) { return round_up(m, 32) * round_up(k, KSTEP); }
+float *frag_scales(void *xf, size_t m, size_t k) {
+  return reinterpret_cast<float *>(static_cast<_Float16 *>(xf) + frag_halfs(m, k));
 }
 
-}  // namespace
-
-float *rows_frag_scales(void *xf, size_t m, size_t k, bool split) {
-  return reinterpret_cast<float *>(static_cast<_Float16 *>(xf) + frag_halfs(m, k, split));
+dim3 grid_of(const RowsGemm &g, const Shape &o, size_t m) {
+  return dim3((unsigned)cdiv(g.n, (size_t)(32 * o.nt)), (unsigned)cdiv(m, (size_t)(32 * o.mt)),
+              (unsigned)o.kz);
 }
-
-namespace {
-
-template <int FMT, int MT, int NT, bool SPLIT>
+template <int FMT>
 void go(const RowsGemm &g, const Shape &o, const void *xf, size_t m, float *y, size_t ldy,
-        size_t zs, hipStream_t s) {
-  const dim3 grid((unsigned)cdiv(g.n, (size_t)(32 * NT)), (unsigned)cdiv(m, (size_t)(32 * MT)),
-                  (unsigned)o.kz);
-  const float *rowmul = rows_frag_scales(const_cast<void *>(xf), m, g.k, SPLIT);
-  hipLaunchKernelGGL((k_rows_gemm<FMT, MT, NT, SPLIT>), grid, dim3(RNT), 0, s,
-                     static_cast<const u32x4 *>(g.W), g.Wd, (int)g.n, g.blocks,
-                     static_cast<const f16x8 *>(xf), rowmul, (int)m, (int)cdiv(g.k, KSTEP), o.per,
-                     y, (int)ldy, zs);
-}
-template <int FMT, bool SPLIT>
-void go_fmt(const RowsGemm &g, const Shape &o, const void *xf, size_t m, float *y, size_t ldy,
-            size_t zs, hipStream_t s) {
-  if (o.mt == 1 && o.nt == 1) go<FMT, 1, 1, SPLIT>(g, o, xf, m, y, ldy, zs, s);
-  else if (o.mt == 1) go<FMT, 1, 2, SPLIT>(g, o, xf, m, y, ldy, zs, s);
-  else if (SPLIT || o.nt == 1) go<FMT, 2, 1, SPLIT>(g, o, xf, m, y, ldy, zs, s);
-  else if constexpr (!SPLIT) go<FMT, 2, 2, SPLIT>(g, o, xf, m, y, ldy, zs, s);
+        hipStream_t s) {
+  const auto kern = o.mt == 1 ? (o.nt == 1 ? k_rows_gemm<FMT, 1, 1> : k_rows_gemm<FMT, 1, 2>)
+                              : (o.nt == 1 ? k_rows_gemm<FMT, 2, 1> : k_rows_gemm<FMT, 2, 2>);
+  hipLaunchKernelGGL(kern, grid_of(g, o, m), dim3(RNT), 0, s, static_cast<const u32x4 *>(g.W),
+                     g.Wd, (int)g.n, g.blocks, static_cast<const f16x8 *>(xf),
+                     frag_scales(const_cast<void *>(xf), m, g.k), (int)m,
+                     (int)cdiv(g.k, KSTEP), o.per, y, (int)ldy);
 }
 
 }  // namespace
 
-size_t rows_frag_bytes(size_t m, size_t k, bool split) {
-  return frag_halfs(m, k, split) * 2 + round_up(m, 32) * sizeof(float);
+size_t rows_frag_bytes(size_t m, size_t k) {
+  return frag_halfs(m, k) * 2 + round_up(m, 32) * sizeof(float);
 }
+
+size_t rows_parts_bytes(size_t m, size_t k) { return round_up(m, 32) * k * 6; }
 
 // Where the line to the tiled kernels lies (whole calls, us, here against
 // tiled).
@@ -519,23 +650,37 @@ bool rows_gemm_fits(int fmt, bool q8_exact, size_t m, size_t n, size_t k) {
 // More than two f32 adds into a cleared element depend on their order; two do
 // not.  Where the tiled kernels take at most two K splits (128 tiles of 128 x
 // 128), so does this one, and the bits of such a call repeat
-int rows_gemm_splits(const RowsGemm &g, size_t m, bool split) {
-  const bool repeats = !split && cdiv(g.n, 128) * cdiv(m, 128) >= 128;
-  return shape_of(g, m, repeats ? 2 : kRowsMaxSplit, split).kz;
+int rows_gemm_splits(const RowsGemm &g, size_t m) {
+  const bool repeats = cdiv(g.n, 128) * cdiv(m, 128) >= 128;
+  return shape_of(g, m, repeats ? 2 : kRowsMaxSplit, false).kz;
+}
+int rows_parts_splits(const RowsGemm &g, size_t m) {
+  return shape_of(g, m, kRowsMaxSplit, true).kz;
 }
 
-syn_status_t launch_rows_frag(int fmt, const float *x, size_t ldx, size_t m, size_t k, bool split,
-                              void *xf, float *y0, size_t ldy, size_t ny, hipStream_t s) {
+syn_status_t launch_rows_frag(int fmt, const float *x, size_t ldx, size_t m, size_t k, void *xf,
+                              float *y0, size_t ldy, size_t ny, hipStream_t s) {
   if (ldx % 4 || k % 8) {
     set_error("GEMM activation stride must be a multiple of 4 floats and K of 8");
     return SYN_ERR_SHAPE_MISMATCH;
   }
-  float *rowmul = rows_frag_scales(xf, m, k, split);
-  const auto kern = nibble_order(fmt) ? (split ? k_rows_frag<true, true> : k_rows_frag<true, false>)
-                                      : (split ? k_rows_frag<false, true> : k_rows_frag<false, false>);
+  const auto kern = nibble_order(fmt) ? k_rows_frag<true> : k_rows_frag<false>;
   hipLaunchKernelGGL(kern, dim3((unsigned)round_up(m, 32)), dim3(FNT), 0, s, x, (int)ldx, (int)m,
-                     (int)k, (int)cdiv(k, KSTEP), static_cast<f16x8 *>(xf), rowmul, y0, (int)ldy,
-                     (int)ny);
+                     (int)k, (int)cdiv(k, KSTEP), static_cast<f16x8 *>(xf), frag_scales(xf, m, k),
+                     y0, (int)ldy, (int)ny);
+  SYN_LAUNCH_CHECK();
+  return SYN_OK;
+}
+
+syn_status_t launch_rows_parts(const float *x, size_t ldx, size_t m, size_t k, void *xf,
+                               hipStream_t s) {
+  if (ldx % 4 || k % 32) {
+    set_error("GEMM activation stride must be a multiple of 4 floats and K of 32");
+    return SYN_ERR_SHAPE_MISMATCH;
+  }
+  const dim3 grid((unsigned)cdiv(k / 8, 256), (unsigned)round_up(m, 32));
+  hipLaunchKernelGGL(k_rows_parts, grid, dim3(256), 0, s, x, (int)ldx, (int)m, (int)(k / 8),
+                     static_cast<bf16x8 *>(xf));
   SYN_LAUNCH_CHECK();
   return SYN_OK;
 }
@@ -544,20 +689,25 @@ syn_status_t launch_rows_gemm(const RowsGemm &g, const void *xf, size_t m, int k
                               size_t ldy, hipStream_t s) {
   const Shape o = shape_of(g, m, kz, false);
   switch (g.fmt) {
-    case SYN_HIP_FMT_Q4_0: go_fmt<SYN_HIP_FMT_Q4_0, false>(g, o, xf, m, y, ldy, 0, s); break;
-    case SYN_HIP_FMT_Q8_0: go_fmt<SYN_HIP_FMT_Q8_0, false>(g, o, xf, m, y, ldy, 0, s); break;
-    case SYN_HIP_FMT_Q4_K: go_fmt<SYN_HIP_FMT_Q4_K, false>(g, o, xf, m, y, ldy, 0, s); break;
-    case SYN_HIP_FMT_Q6_K: go_fmt<SYN_HIP_FMT_Q6_K, false>(g, o, xf, m, y, ldy, 0, s); break;
+    case SYN_HIP_FMT_Q4_0: go<SYN_HIP_FMT_Q4_0>(g, o, xf, m, y, ldy, s); break;
+    case SYN_HIP_FMT_Q8_0: go<SYN_HIP_FMT_Q8_0>(g, o, xf, m, y, ldy, s); break;
+    case SYN_HIP_FMT_Q4_K: go<SYN_HIP_FMT_Q4_K>(g, o, xf, m, y, ldy, s); break;
+    case SYN_HIP_FMT_Q6_K: go<SYN_HIP_FMT_Q6_K>(g, o, xf, m, y, ldy, s); break;
     default: return SYN_ERR_INVALID_ARG;
   }
   SYN_LAUNCH_CHECK();
   return SYN_OK;
 }
 
-syn_status_t launch_rows_gemm_split(const RowsGemm &g, const void *xf, size_t m, int kz, float *y,
+syn_status_t launch_rows_gemm_parts(const RowsGemm &g, const void *xf, size_t m, int kz, float *y,
                                     size_t ldy, size_t zs, hipStream_t s) {
-  if (g.fmt != SYN_HIP_FMT_Q4_0 || (kz > 1 && zs == 0)) return SYN_ERR_INVALID_ARG;
-  go_fmt<SYN_HIP_FMT_Q4_0, true>(g, shape_of(g, m, kz, true), xf, m, y, ldy, zs, s);
+  if (g.fmt != SYN_HIP_FMT_Q4_0 || g.k % 32) return SYN_ERR_INVALID_ARG;
+  const Shape o = shape_of(g, m, kz, true);
+  const auto kern = o.mt == 1 ? (o.nt == 1 ? k_rows_gemm_parts<1, 1, 4> : k_rows_gemm_parts<1, 2, 4>)
+                              : (o.nt == 1 ? k_rows_gemm_parts<2, 1, 3> : k_rows_gemm_parts<2, 2, 2>);
+  hipLaunchKernelGGL(kern, grid_of(g, o, m), dim3(RNT), 0, s, static_cast<const uint2 *>(g.W),
+                     g.Wd, (int)g.n, g.blocks, static_cast<const bf16x8 *>(xf), (int)m, 2 * o.per,
+                     y, (int)ldy, zs);
   SYN_LAUNCH_CHECK();
   return SYN_OK;
 }

@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 import oracle as O
+from perf import cases
 from synapse_amd import hip
 
 pytestmark = pytest.mark.gpu
@@ -86,3 +87,21 @@ def test_generate_after_a_prompt_and_full_cache():
     with pytest.raises(hip.SynapseError):
         g.prefill(O.token_ids(49, 1, cfg["vocab"]))
     g.close()
+
+
+# the row products round nothing before their f32 sums and have no sum to cancel (the step takes
+# 8 sum(x) off every block): their logits are less than half as far from float64 as the step's
+@pytest.mark.parametrize("prompt", [9, 64])
+def test_prompt_rows_error_against_float64(prompt):
+    case = dict(kind="lm", model="hybrid", layers=4, vocab=32000, prompt=prompt, steps=0)
+    state = cases.prepare(case, 1)
+    lm, ids = state["lm"], state["ids"]
+    want = cases.exact(case, 1)[0]
+    rows = lm.prefill(ids)
+    lm.reset()
+    for t in ids:
+        step = lm.decode_one(int(t))
+    err = [float(np.linalg.norm(v - want) / np.linalg.norm(want)) for v in (rows, step)]
+    print("prompt", prompt, "rows", err[0], "step", err[1], flush=True)
+    assert err[0] <= 0.5 * err[1], err
+    lm.close()
