@@ -105,3 +105,27 @@ def test_prompt_rows_error_against_float64(prompt):
     print("prompt", prompt, "rows", err[0], "step", err[1], flush=True)
     assert err[0] <= 0.5 * err[1], err
     lm.close()
+
+
+# the rows kernels' most tokens at once, then the rest of the prompt token by token
+def test_prompt_past_the_rows_limit():
+    cfg = dict(BASE, n_layers=2, layer_kinds=[0, 1], max_seq=2070)
+    g = hip.HybridLM(cfg)
+    g.init_synthetic(std=0.06)
+    ids = O.token_ids(2052, 0x5EED0000 + 0xFFFF, cfg["vocab"])
+    loop = [g.decode_one(int(t)) for t in ids]
+    for n in (2047, 2048, 2049, 2051):
+        g.reset()
+        got = g.prefill(ids[:n])
+        assert g.pos == n
+        after = g.decode_one(int(ids[n]))
+        worst = max(_rel(got, loop[n - 1]), _rel(after, loop[n]))
+        print("n", n, "worst", worst, flush=True)
+        assert worst <= TOL, (n, worst)
+    for n in (2048, 2049):
+        g.reset()
+        toks, margins = g.generate(ids[:n], 1)
+        top = np.sort(loop[n - 1])[-2:]
+        assert top[1] - top[0] < 1e-3 or int(toks[0]) == int(np.argmax(loop[n - 1]))
+        assert abs(float(margins[0]) - float(top[1] - top[0])) < 1e-3
+    g.close()

@@ -13,6 +13,8 @@ pytestmark = pytest.mark.gpu
 TINY = dict(d_model=64, d_inner=128, d_state=16, d_conv=4, dt_rank=8, n_layers=2, vocab=256)
 RAGGED = dict(d_model=72, d_inner=136, d_state=16, d_conv=3, dt_rank=12, n_layers=3, vocab=301)
 WIDE = dict(d_model=1024, d_inner=2048, d_state=16, d_conv=4, dt_rank=64, n_layers=2, vocab=512)
+# a block of 512 tokens fills 256 tiles of 128 x 128 in in_proj
+BROAD = dict(d_model=256, d_inner=4096, d_state=16, d_conv=4, dt_rank=32, n_layers=1, vocab=256)
 # shapes the row kernels do not take: the token loop serves the prompt
 SHORT_STATE = dict(TINY, d_state=8)
 
@@ -31,8 +33,9 @@ def _bits(a):
 # 512 tokens and one more
 @pytest.mark.parametrize("cfg,lengths", [(TINY, (2, 3, 4, 5, 16, 17, 33, 65, 512, 513)),
                                          (RAGGED, (3, 16, 31, 32, 130)),
-                                         (WIDE, (8, 64, 70)), (SHORT_STATE, (5, 20))],
-                         ids=["tiny", "ragged", "wide", "short_state"])
+                                         (WIDE, (8, 64, 70)), (BROAD, (512,)),
+                                         (SHORT_STATE, (5, 20))],
+                         ids=["tiny", "ragged", "wide", "broad", "short_state"])
 @pytest.mark.parametrize("xdt", [False, True], ids=["ref", "int8xdt"])
 @pytest.mark.parametrize("fused", [True, False], ids=["fused", "unfused"])
 def test_prompt_rows_equal_the_token_loop(cfg, lengths, xdt, fused):

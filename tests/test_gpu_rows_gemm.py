@@ -296,3 +296,36 @@ def test_q4_0_rows_capture_and_streams():
     for y, v in zip(ys, want):
         assert torch.equal(y, v)
     lin.close()
+
+
+# 64 columns a workgroup (over 8192), a part of the last one, one and two tiles of 32 rows, block
+# counts that leave half a step over
+@pytest.mark.parametrize("fmt", sorted(EL), ids=lambda f: NAME[f])
+@pytest.mark.parametrize("n", [8196, 14340])
+def test_rows_gemm_wide(fmt, n):
+    k = 512 if EL[fmt] == 256 else 288
+    lin, w = _linear(fmt, n, k, n)
+    x = np.random.default_rng(n).standard_normal((64, k)).astype(np.float32)
+    for m in (9, 16, 17, 32, 33, 64):
+        _check(lin, w, x[:m], fmt == hip.FMT_Q4_0 and m <= 16)
+    lin.close()
+
+
+# rows of y that are no whole 16 bytes, or start off them, are not cleared 16 bytes at a time
+@pytest.mark.parametrize("n,offset", [(1021, 0), (1024, 1), (1022, 3)])
+def test_k_split_unaligned_output(n, offset):
+    m, k = 24, 4096
+    lin, w = _linear(hip.FMT_Q8_0, n, k, n)
+    x = np.random.default_rng(n).standard_normal((m, k)).astype(np.float32)
+    bx, by = hip.DeviceBuffer.from_array(x), hip.DeviceBuffer(4 * (m * n + 8))
+    by.upload(np.full(m * n + 8, 7, np.float32))
+    lin.forward_dev(m, bx.ptr, by.ptr + 4 * offset)
+    hip.check(hip.lib().syn_hip_stream_synchronize(None))
+    y = by.download(m * n + 8, np.float32)
+    got = y[offset:offset + m * n].reshape(m, n).astype(np.float64)
+    size = np.abs(x).astype(np.float64) @ np.abs(w).T
+    assert (np.abs(got - x.astype(np.float64) @ w.T) / size).max() <= 2.0**-10 * (1 + 2.0**-4)
+    assert (y[:offset] == 7).all() and (y[offset + m * n:] == 7).all()
+    for b in (bx, by):
+        b.close()
+    lin.close()

@@ -72,3 +72,24 @@ def test_full_softmax_stream(n, scale):
     x = (np.random.default_rng(n).standard_normal(n) * scale).astype(np.float32)
     _check(x, draws=6, temperature=1.0)
     _check(x, draws=3, temperature=1.0, top_p=0.6)
+
+
+# NaN logits leave the group maxima for the general route; infinite ones do not
+@pytest.mark.parametrize("n", [5, 64, 700, 5000, 30000])
+def test_nan_and_infinite_logits(n):
+    rng = np.random.default_rng(n)
+    base = (rng.standard_normal(n) * 3).astype(np.float32)
+    both = base.copy()
+    both[0], both[n // 2] = np.nan, np.inf
+    for x in (both, np.full(n, np.nan, np.float32)):
+        for kw in (dict(temperature=0.9, top_k=3),
+                   dict(temperature=0.8, top_k=40, top_p=0.9, repetition_penalty=1.2)):
+            _check(x, (1, 2, 1), **kw)
+    ends = base.copy()
+    ends[[0, n - 1]] = np.inf
+    half = base.copy()
+    half[:n // 2] = -np.inf
+    for x in (ends, half):
+        for kw in (dict(temperature=0.0), dict(temperature=0.9), dict(temperature=0.9, top_k=3),
+                   dict(temperature=0.7, top_p=0.6)):
+            _check(x, (1, 2, 1), **kw)
