@@ -130,6 +130,12 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef long long i64x2 __attribute__((ext_vector_type(2)));
 
+// the 8-bit level of v for inv = 127 / max|x| of its row (quantize.zig:12-47)
+__device__ __forceinline__ int8_t q8_level(float v, float inv) {
+  const float r = roundf(v * inv);
+  return (int8_t)(int)fminf(127.0f, fmaxf(-127.0f, r));
+}
+
 // 4 x 4 transpose between the four groups of 16 lanes and the elements of v:
 // element g of group s goes to element s of group g
 __device__ __forceinline__ f32x4 groups_transposed(f32x4 v) {

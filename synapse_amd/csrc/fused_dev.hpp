@@ -67,11 +67,7 @@ __device__ float quantize_regs_with_max(const float (&v)[R], int n, float mx, in
 #pragma unroll
   for (int u = 0; u < R; u++) {
     const int j = threadIdx.x + u * NT;
-    if (j < n) {
-      float r = roundf(v[u] * inv);
-      r = fminf(127.0f, fmaxf(-127.0f, r));
-      q[j] = (int8_t)(int)r;
-    }
+    if (j < n) q[j] = q8_level(v[u], inv);
   }
   return mx / 127.0f;
 }
@@ -296,11 +292,7 @@ __device__ float quantize_range_with_max(const float (&v)[R], int k0, int k1, fl
 #pragma unroll
   for (int u = 0; u < R; u++) {
     const int j = k0 + tid + u * NT;
-    if (j < k1) {
-      float r = roundf(v[u] * inv);
-      r = fminf(127.0f, fmaxf(-127.0f, r));
-      xq[j] = (int8_t)(int)r;
-    }
+    if (j < k1) xq[j] = q8_level(v[u], inv);
   }
   return mx / 127.0f;
 }

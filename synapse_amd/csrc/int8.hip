@@ -20,13 +20,7 @@
 namespace syn {
 
 // --------------------------------------------------------------- quantizer
-// one workgroup per row; max|x| is order-free, the rest is elementwise.  The
-// value's 8-bit level for inv = 127 / max (quantize.zig:12-47)
-__device__ __forceinline__ int8_t q8_level(float v, float inv) {
-  float r = roundf(v * inv);
-  r = fminf(127.0f, fmaxf(-127.0f, r));
-  return (int8_t)(int)r;
-}
+// one workgroup per row; max|x| is order-free, the rest is elementwise
 __device__ __forceinline__ uint32_t q8_pack(const float4 &v, float inv) {
   return (uint32_t)(uint8_t)q8_level(v.x, inv) | (uint32_t)(uint8_t)q8_level(v.y, inv) << 8 |
          (uint32_t)(uint8_t)q8_level(v.z, inv) << 16 | (uint32_t)(uint8_t)q8_level(v.w, inv) << 24;

@@ -90,11 +90,7 @@ __device__ void quantize_row_lds(const float *v, int n, int8_t *q, float *scale_
     return;
   }
   const float inv = 127.0f / mx;
-  for (int j = threadIdx.x; j < n; j += blockDim.x) {
-    float r = roundf(v[j] * inv);
-    r = fminf(127.0f, fmaxf(-127.0f, r));
-    q[j] = (int8_t)(int)r;
-  }
+  for (int j = threadIdx.x; j < n; j += blockDim.x) q[j] = q8_level(v[j], inv);
   if (threadIdx.x == 0) *scale_out = mx / 127.0f;
 }
 

@@ -91,11 +91,7 @@ __global__ void __launch_bounds__(256)
     return;
   }
   const float inv = 127.0f / mx;
-  for (int j = threadIdx.x; j < H; j += blockDim.x) {
-    float r = roundf(sm[j] * inv);
-    r = fminf(127.0f, fmaxf(-127.0f, r));
-    xq[j] = (int8_t)(int)r;
-  }
+  for (int j = threadIdx.x; j < H; j += blockDim.x) xq[j] = q8_level(sm[j], inv);
   if (threadIdx.x == 0) *sx = mx / 127.0f;
 }
 
@@ -407,11 +403,7 @@ __global__ void __launch_bounds__(256)
     float mx = fabsf(v);
     for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
     int8_t q = 0;
-    if (mx != 0.0f && tid < dr) {
-      float r = roundf(v * (127.0f / mx));
-      r = fminf(127.0f, fmaxf(-127.0f, r));
-      q = (int8_t)(int)r;
-    }
+    if (mx != 0.0f && tid < dr) q = q8_level(v, 127.0f / mx);
     reinterpret_cast<int8_t *>(xq4)[tid] = q;
     if (tid == 0) s_q = mx == 0.0f ? 1.0f : mx / 127.0f;
   }

@@ -38,11 +38,7 @@ __device__ __forceinline__ void quantize_lds_row(const float *v, int n, float mx
     return;
   }
   const float inv = 127.0f / mx;
-  for (int j = threadIdx.x; j < n; j += kRowNT) {
-    float r = roundf(v[j] * inv);
-    r = fminf(127.0f, fmaxf(-127.0f, r));
-    q[j] = (int8_t)(int)r;
-  }
+  for (int j = threadIdx.x; j < n; j += kRowNT) q[j] = q8_level(v[j], inv);
   if (threadIdx.x == 0) *scale = mx / 127.0f;
 }
 
@@ -196,11 +192,7 @@ __global__ void __launch_bounds__(256)
       float mx = fabsf(v);
       for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
       int8_t q = 0;
-      if (mx != 0.0f && lane < dr) {
-        float r = roundf(v * (127.0f / mx));
-        r = fminf(127.0f, fmaxf(-127.0f, r));
-        q = (int8_t)(int)r;
-      }
+      if (mx != 0.0f && lane < dr) q = q8_level(v, 127.0f / mx);
       reinterpret_cast<int8_t *>(xq[j])[lane] = q;
       if (lane == 0) sq[j] = mx == 0.0f ? 1.0f : mx / 127.0f;
     }
