@@ -432,8 +432,8 @@ struct syn_hip_hlm_s {
   static constexpr size_t kRowsMax = 2048;
   // Below this many tokens the replayed step is the faster form: a layer of
   // the rows form takes ~65 us at 3-32 tokens, the step ~20 us a token.  LFM2.5
-  // widths, four layers, whole calls: 3 tokens 311 us against 495, 64 tokens
-  // 394 against 9400
+  // widths, four layers, whole calls: 3 tokens 361 us against 495, 64 tokens
+  // 356 against 9400
   static constexpr size_t kRowsMin = 3;
   struct RowsScratch {
     size_t cap = 0;
@@ -509,7 +509,9 @@ struct syn_hip_hlm_s {
                                 stream));
       HRows p;
       if (Ly.kind == 0) {
-        SYN_TRY(rows_gemm(Ly.in, n, kRowsMaxSplit, &p));
+        // (the conv reads the splits of B and x once per tap: two splits cost it
+        // the 1.8 us that they save the product)
+        SYN_TRY(rows_gemm(Ly.in, n, 1, &p));
         SYN_TRY(launch_hrows_conv(p, Ly.conv_w.as<float>(),
                                   c.conv_bias ? Ly.conv_b.as<float>() : nullptr, T, (int)I,
                                   (int)ck, Ly.conv_state.as<float>() + (n & 1) * I * ck, rs.xf.p,

@@ -326,10 +326,9 @@ __global__ void __launch_bounds__(RNT) __attribute__((amdgpu_waves_per_eu(2, 2))
 // holds dwords 0 and 1 of a block's levels, the others 2 and 3, so the
 // activations of MFMA j are elements 8 (2 lh + j) .. +7.  PF steps in flight.
 // Bound by the activations' way from L2, six bytes an element for every tile of
-// columns: 64 rows, the four projections of an LFM2.5 conv layer, 64 columns a
-// workgroup where that is a round of workgroups (a prompt of 64 tokens and four
-// layers 394 us, 512 tokens 908; 412 and 978 with 32 columns, 374 and 840 with
-// operands of two f16, which round the activations to 22 bits).
+// columns (1024 -> 13312, 64 rows 14.5 us, 512 rows 81), and on small grids by a
+// wave's chain of loads and MFMAs (1024 -> 1024, 64 rows 6.2 us).  Operands of two
+// f16, which round the activations to 22 bits, took 13.9, 71.6 and 7.0.
 // grid (ceil(N / 32 NT), ceil(M / 32 MT), K splits); split z writes y + z zs
 template <int MT, int NT, int PF>
 __global__ void __launch_bounds__(RNT) __attribute__((amdgpu_waves_per_eu(2, 2)))
@@ -407,7 +406,9 @@ __global__ void __launch_bounds__(RNT) __attribute__((amdgpu_waves_per_eu(2, 2))
   if (b < s1) {
 #pragma unroll
     for (int u = 0; u < PF; u++) {
-      load(st[u], min(b + u * RW, s1 - 1));
+      // a wave of a short K has fewer steps than that (with 64 x 64 tiles it has
+      // not, and the branch would cost registers)
+      if (MT * NT == 4 || b + u * RW < s1) load(st[u], min(b + u * RW, s1 - 1));
       hold();
     }
     for (bool more = true; more;) {
@@ -548,26 +549,28 @@ __global__ void __launch_bounds__(256)
   parts_put(xf, chunks >> 2, m, c, v);
 }
 
-
 // Columns per workgroup and K splits (at least two steps per wave) with the
 // least time by this count, in steps of a 32-column wave (~0.8 us each): 256
 // CUs take one workgroup at a time, a workgroup costs four steps beside its
 // own, a step of 64 columns 1.75 of 32, and 250,000 atomic adds of K splits
 // one.  (8192 -> 2048, Q8_0: 256 rows 24.0 us in 256 workgroups of 32 columns,
 // 512 rows 36.6 in 256 of 64; 384 rows 39.0 in 384 of 32, 31.7 in 192 of 64.
-// 3072 -> 3072, 384 rows: 27 us in 288 of 64, 35 in two splits of them.)
+// 3072 -> 3072, 384 rows: 27 us in 288 of 64, 35 in two splits of them.)  parts:
+// one tile of 32 rows a workgroup while that is one round of workgroups (64 rows,
+// 1024 -> 3072 6.3 us, with two tiles 9.2), and K splits down to one such step, two
+// blocks, per wave (16 rows, 1024 -> 1024 4.4 us in two, 6.0 unsplit).
 struct Shape {
   int mt, nt, kz, per;
 };
 Shape shape_of(const RowsGemm &g, size_t m, int kz_max, bool parts) {
   Shape o{};
   const int steps = (int)cdiv(g.k, KSTEP);
-  o.mt = m > 32 ? 2 : 1;
+  o.mt = m > 32 && !(parts && cdiv(g.n, 32) * cdiv(m, 32) <= 256) ? 2 : 1;
   const int tiles_m = (int)cdiv(m, (size_t)(32 * o.mt));
   float best = 0.0f;
   for (int nt = 1; nt <= 2; nt++) {
     const size_t tiles = cdiv(g.n, (size_t)(32 * nt)) * tiles_m;
-    for (int kz = 1; kz <= std::min(kz_max, std::max(1, steps / (2 * RW))); kz++) {
+    for (int kz = 1; kz <= std::min(kz_max, std::max(1, steps / (parts ? RW : 2 * RW))); kz++) {
       const float own = (float)cdiv((size_t)steps, (size_t)(RW * kz)) * (nt == 2 ? 1.75f : 1.0f);
       const float adds = kz > 1 ? (float)m * (float)g.n * (float)kz / 250000.0f : 0.0f;
       const float cost = (float)cdiv(tiles * kz, 256) * (4.0f + own) + adds;
