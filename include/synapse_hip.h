@@ -233,10 +233,8 @@ typedef struct {
  * d_logits f32 [vocab] (not modified), d_history the generated tokens
  * [n_history], u the draw rng.gen::<f32>() the reference would take.  The
  * token goes to d_token (device), asynchronously on `stream`.  d_status
- * (device, nullable) gets 0, or 1 when top-p would have to sort more than
- * 4096 candidates (top-p without top-k over a large vocabulary; the token is
- * then 0).  No counterpart in the reference's C ABI (sampling runs in Rust
- * there). */
+ * (device, nullable) gets 0.  No counterpart in the reference's C ABI
+ * (sampling runs in Rust there). */
 syn_status_t syn_hip_sample(const float *d_logits, size_t vocab, const uint32_t *d_history,
                             size_t n_history, const syn_hip_sampler *params, float u,
                             uint32_t *d_token, int *d_status, void *stream);

@@ -23,8 +23,9 @@
 //   mamba.hip).
 //
 // The reference prefills on the CPU with f32 weights and then decodes on the
-// GPU (examples/lfm25_inference.rs:86-99); this decoder feeds a prompt
-// through the decode step (Q4 weights), one token at a time.
+// GPU (examples/lfm25_inference.rs:86-99); this decoder runs a prompt into an
+// empty cache over all its tokens at once (hlm_prefill.hip, Q4 weights), and
+// the rest of a longer one or a later prompt through the decode step.
 #include <algorithm>
 #include <cmath>
 #include <thread>
