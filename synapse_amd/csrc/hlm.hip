@@ -245,6 +245,9 @@ struct syn_hip_hlm_s {
   // residual r [H], the split-K accumulator of in_proj / q|k|v (cleared by
   // the projection after its reader), attention chunk partials, lm_head top-2
   bool use_fused = true, fused_ok = false;
+  // the step saturates its fixed-point sums at 2^27, which weights of wide block
+  // scales reach; a prompt of such a model goes token by token
+  bool wide = false;
   KqfPlan fp_in, fp_out, fp_qkv, fp_o, fp_gu, fp_down;
   DevBuf f_r, f_acc, f_ao, f_aml, f_pv, f_pi, f_pv2;
   size_t n_qkv = 0;
@@ -259,15 +262,17 @@ struct syn_hip_hlm_s {
   // st()->pos; logits -> argmax -> st()->token, pos += 1
   // the fused step's plans and buffers, when every shape fits its kernels
   syn_status_t setup_fused() {
-    fused_ok = false;
+    fused_ok = wide = false;
     const int fm[1] = {SYN_HIP_FMT_Q4_0};
     if (!kqf_fits((int)H, (int)qd, (int)F, (int)nh, (int)nkv, (int)hd, (int)S, fm, 1) ||
         I % 256 || !head_f32_fits((int)H))
       return SYN_OK;
     bool any_conv = false, any_gqa = false;
     for (auto &Ly : layers) {
-      for (QLinearQ4_0 *q : {&Ly.in, &Ly.out, &Ly.qkv, &Ly.o, &Ly.gu, &Ly.down})
+      for (QLinearQ4_0 *q : {&Ly.in, &Ly.out, &Ly.qkv, &Ly.o, &Ly.gu, &Ly.down}) {
         if (q->n && !q->gemm_ok()) return SYN_OK;  // halved subnormal scales
+        if (q->n && q->has_wide_scale) wide = true;
+      }
       (Ly.kind == 0 ? any_conv : any_gqa) = true;
     }
     const Layer *conv = nullptr, *gqa = nullptr;
@@ -446,7 +451,7 @@ struct syn_hip_hlm_s {
   // row kernels' registers and the prompt attention's LDS
   bool rows_supported() const {
     return use_fused && fused_ok && H <= (size_t)kHrowsMaxH && I <= (size_t)kHrowsMaxH &&
-           qd <= (size_t)kHrowsMaxH && F <= (size_t)kHrowsMaxF;
+           qd <= (size_t)kHrowsMaxH && F <= (size_t)kHrowsMaxF && !wide;
   }
   static RowsGemm rows_of(const QLinearQ4_0 &q) {
     RowsGemm g;

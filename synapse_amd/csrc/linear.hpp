@@ -126,6 +126,7 @@ struct QLinearQ4_0 {
   // reference's GGUF Q4_0 path; false = the Zig GEMV's IEEE conversion
   bool rs_f16_scales = false;
   bool has_subnormal_scale = false;  // some block scale is an f16 subnormal (set at upload)
+  bool has_wide_scale = false;       // some |block scale| is 2^13 or more, or not finite
   DevBuf xh;                         // f16 activations for the MFMA GEMM
   size_t xh_bytes = 0;  // its size (f16_rows_bytes)
   SplitKSlots sk;  // gemv()'s one-launch K split (split_k.hpp)

@@ -607,7 +607,7 @@ syn_status_t QLinearQ4_0::upload_packed(const uint8_t *packed, size_t n_, size_t
   const size_t P = cdiv(n_, 64), B = (size_t)blocks;
   std::vector<uint8_t> hn(P * B * 64 * 16, 0x88);  // padding rows: nibble 8 -> value 0
   std::vector<uint16_t> hs(P * B * 64, 0);
-  has_subnormal_scale = false;
+  has_subnormal_scale = has_wide_scale = false;
   for (size_t row = 0; row < n_; row++) {
     const size_t p = row / 64, r = row % 64;
     for (size_t b = 0; b < B; b++) {
@@ -615,6 +615,7 @@ syn_status_t QLinearQ4_0::upload_packed(const uint8_t *packed, size_t n_, size_t
       const uint16_t d = (uint16_t)(src[0] | (src[1] << 8));
       hs[(p * B + b) * 64 + r] = d;
       if ((d & 0x7c00u) == 0 && (d & 0x3ffu) != 0) has_subnormal_scale = true;
+      if ((d & 0x7fffu) > 0x6fffu) has_wide_scale = true;
       std::memcpy(&hn[((p * B + b) * 64 + r) * 16], src + 2, 16);
     }
   }

@@ -129,3 +129,18 @@ def test_prompt_past_the_rows_limit():
         assert top[1] - top[0] < 1e-3 or int(toks[0]) == int(np.argmax(loop[n - 1]))
         assert abs(float(margins[0]) - float(top[1] - top[0])) < 1e-3
     g.close()
+
+
+# weights whose block scales reach 2^13 (standard deviation 3e4): the step's sums saturate, and a
+# prompt follows it, token by token
+def test_wide_block_scales_follow_the_step():
+    cfg = dict(BASE, n_layers=2, layer_kinds=[0, 1], max_seq=40)
+    g = hip.HybridLM(cfg)
+    g.init_synthetic(std=3e4)
+    ids = O.token_ids(12, 0x5EED0000 + 0xFFFF, cfg["vocab"])
+    for t in ids:
+        want = g.decode_one(int(t))
+    g.reset()
+    got = g.prefill(ids)
+    np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))
+    g.close()
