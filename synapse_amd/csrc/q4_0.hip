@@ -551,6 +551,16 @@ syn_status_t QLinearQ4_0::gemv(size_t m, const float *d_x, size_t ldx, float *d_
 syn_status_t QLinearQ4_0::rows16(size_t m, const float *d_x, size_t ldx, float *d_y, size_t ldy,
                                  hipStream_t s) {
   SYN_TRY(ensure_slots());
+  if (rows_overlap(d_x, m, k, ldx, d_y, n, ldy)) {  // every workgroup reads all of x
+    const size_t bytes = ((m - 1) * ldx + k) * sizeof(float);
+    if (xh_bytes < bytes) {
+      SYN_HIP(hipDeviceSynchronize());
+      SYN_TRY(xh.alloc(bytes));
+      xh_bytes = bytes;
+    }
+    SYN_HIP(hipMemcpyAsync(xh.p, d_x, bytes, hipMemcpyDeviceToDevice, s));
+    d_x = xh.as<float>();
+  }
   const Rows16Plan o = rows16_plan(n, blocks);
   const auto kern = o.nt == 2 ? k_rows16_q4_0<2> : k_rows16_q4_0<4>;
   hipLaunchKernelGGL(kern, dim3(o.tiles, o.ks), dim3(64 * kRows16Waves), 0, s, nib.as<u32x4>(),

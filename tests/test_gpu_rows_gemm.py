@@ -329,3 +329,23 @@ def test_k_split_unaligned_output(n, offset):
     for b in (bx, by):
         b.close()
     lin.close()
+
+
+# y over x, and from x's second row on
+@pytest.mark.parametrize("n,k", [(2048, 2048), (8224, 4096)])
+@pytest.mark.parametrize("row", [0, 1])
+def test_q4_0_rows_in_place(n, k, row):
+    m = 12
+    lin, _ = _raw(hip.FMT_Q4_0, n, k, 5)
+    x = np.random.default_rng(n).standard_normal((m, k)).astype(np.float32)
+    want = lin.forward(x)
+    size = row * k + m * max(n, k)
+    buf = hip.DeviceBuffer(4 * size)
+    for _ in range(3):
+        buf.upload(np.concatenate([x.ravel(), np.zeros(size - m * k, np.float32)]))
+        lin.forward_dev(m, buf.ptr, buf.ptr + 4 * row * k)
+        hip.check(hip.lib().syn_hip_stream_synchronize(None))
+        got = buf.download(size, np.float32)[row * k:row * k + m * n].reshape(m, n)
+        np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))
+    buf.close()
+    lin.close()
